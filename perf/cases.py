@@ -158,3 +158,25 @@ def tolerance(case):
     if case["kind"] == "ffn_bt":
         return {"rel": 1.2e-3, "max": 6e-3}
     return {"rel": 8e-4, "max": 2e-3}
+
+
+def exact(case, seed):
+    # the operator's formula in float64, no rounding between the products of the feed-forward pair
+    st = prepare(case, seed)
+    kind, x = st["kind"], st["x"].double()
+    if kind == "int4":
+        nibbles = torch.stack((st["w"] & 15, st["w"] >> 4), dim=-1)  # even element in the low nibble
+        w = nibbles.flatten(1).double().sub_(8.0)
+    else:
+        w = st["w"].double()
+    sums = x @ (w if kind in ("edgemm", "residual") else w.t())
+    if kind == "ffn_bt":
+        h = torch.nn.functional.gelu(sums + st["b1"].double())
+        return {"h": h, "c": h @ st["w2"].double().t() + st["b2"].double()}
+    if kind == "w8a8":
+        return {"acc": sums.round().int(), "c": sums * st["scale"].double() * st["x_scale"]}
+    if kind in ("int8", "int4"):
+        return sums * st["scale"].double()
+    if kind in ("residual", "residual_bt"):
+        return sums + st["residual"].double()
+    return sums
