@@ -28,6 +28,7 @@ EXT_NAME = "speedgate" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so")
 HIP_SOURCES = [
     "fg_kernels_nk.hip",
     "fg_kernels_kn.hip",
+    "fg_kernels_tile.hip",
     "fg_kernels_i8.hip",
     "fg_kernels_misc.hip",
     "fg_capi.hip",

@@ -72,12 +72,16 @@ int run_gemm(const void* A, const void* W, void* C, int M, int N, int K, int acc
           (size_t)p.grid_x * p.grid_y * p.splitk * p.waves > kWsMailboxFlags) {
         return FG_ERR_UNSUPPORTED;
       }
+      // (beyond 16 rows the partials meet through the counters: launch_tile ignores both flags)
       a.accumulate |= kFlagXcdLocal | (p.fused == 4 ? kFlagPretendForeign : 0);
     }
   }
+  // rows of pitched weights so far apart that a step's offsets leave 32 bits stay with the 16-row kernel
+  const int form = 256ull * ldw < (1ull << 32) ? tile_form(M, N, K, p) : -1;
   (void)hipGetLastError();
   bool ok = false;
-  switch (p.kernel) {
+  if (form >= 0) ok = launch_tile(form, kn, p, a, s);
+  else switch (p.kernel) {
     case FG_KERNEL_NK_DOT2: ok = launch_nk_dot2(p, a, s); break;
     case FG_KERNEL_NK_MFMA4: ok = launch_nk_mfma4(p, a, s); break;
     case FG_KERNEL_NK_MFMA_R: ok = launch_nk_mfma_r(p, a, s); break;

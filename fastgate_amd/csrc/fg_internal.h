@@ -46,6 +46,8 @@ bool launch_nk_mfma4(const fg_plan_t& p, const GemmArgs& a, hipStream_t s);
 bool launch_nk_mfma_r(const fg_plan_t& p, const GemmArgs& a, hipStream_t s);
 bool launch_kn_dot2(const fg_plan_t& p, const GemmArgs& a, hipStream_t s);
 bool launch_kn_mfma(const fg_plan_t& p, const GemmArgs& a, hipStream_t s);
+// More than 16 rows, either layout (kn: W is [K,N]), in form `form` of tile_form().
+bool launch_tile(int form, bool kn, const fg_plan_t& p, const GemmArgs& a, hipStream_t s);
 
 // Second pass of split-K: C[m,n] = fp16( tail( Σ_s ws[s,m,n] (+ C[m,n]) ) ), fixed summation
 // order; `flags` and `bias` as in GemmArgs.

@@ -13,6 +13,16 @@ bool nk_mfma4_supported(int m_block, int tile_n, int unroll);
 bool kn_dot2_supported(int m_block, int unroll);
 bool kn_mfma_supported(int unroll);
 
+// Tiles of the kernel for more than 16 rows (fg_kernels_tile.hip): rows and columns of C per
+// workgroup, k per step.  tile_form returns the id of the form a plan runs in, or -1 for a plan that
+// takes another kernel; [N,K] plans ask for the kernel with m_block 32 and tile_n 64, [K,N] plans
+// of FG_KERNEL_KN_MFMA take it whenever M > 16.
+struct TileForm {
+  int rows, cols, bk;
+};
+bool tile_form_info(int form, TileForm* out);
+int tile_form(int M, int N, int K, const fg_plan_t& p);
+
 // FG_OK, FG_ERR_INVALID_ARG or FG_ERR_ALIGN128.
 int plan_validate_shape(int M, int N, int K, int w_layout);
 // The library's plan (splitk 0) or its plan around a forced split.  Shape already validated.

@@ -33,6 +33,18 @@ bool kn_dot2_supported(int mb, int u) {
 }
 bool kn_mfma_supported(int u) { return u == 1 || u == 2 || u == 4; }
 
+// Forms of the kernel for more than 16 rows; ids as in launch_tile.
+static const TileForm kTileForms[] = {
+    {32, 64, 128}, {32, 128, 128}, {64, 64, 128}, {96, 64, 128}, {128, 64, 128}, {128, 128, 64}, {64, 128, 64},
+};
+constexpr int kTileFormCount = sizeof(kTileForms) / sizeof(kTileForms[0]);
+
+bool tile_form_info(int form, TileForm* out) {
+  if (form < 0 || form >= kTileFormCount) return false;
+  *out = kTileForms[form];
+  return true;
+}
+
 namespace {
 
 // Compute units the rules aim at.  The rules were fitted on 256 (MI355X); the C ABI sets the
@@ -40,6 +52,8 @@ namespace {
 int kCUs = 256;
 int kXccs = 8;
 
+
+bool tile_wins(int M, int N, int K, int w_layout);
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
@@ -68,6 +82,61 @@ int pick_splitk(int tiles, int waves, int items, int M, int N, int K, int target
     if (score > best_score + 1e-9) {
       best_score = score;
       best = S;
+    }
+  }
+  return best;
+}
+
+// Time of a call in a form, us: c + c2 q + steps max(t1, q t2), q workgroups on the busiest CU, `steps`
+// of bk k each; a split adds s0 + s2 S + s1 S M N / 2^20 (partials written and read again).  t1 is
+// what a step takes when a CU has one workgroup (latency), t2 what each takes when several keep it
+// busy.  Fitted, one form and layout at a time, to 4000 timings over sixteen (N, K) from 1024 x 4096 to
+// 28672 x 2048, twelve M from 17 to 256 and splits of 1 .. 16 (8 % rms); the form and split it picks
+// are on average 2 % slower than the best of that sweep.
+struct TileCost {
+  float c, c2, t1, t2, s0, s1, s2;
+};
+const TileCost kTileCosts[2][kTileFormCount] = {
+    {{2.80f, 0.95f, 0.257f, 0.454f, 0.54f, 2.81f, 0.20f},
+     {0.85f, 3.53f, 0.511f, 0.732f, 0.00f, 3.57f, 0.26f},
+     {3.31f, 0.61f, 0.508f, 0.573f, 0.06f, 2.69f, 0.30f},
+     {1.50f, 2.90f, 0.641f, 0.620f, 0.00f, 2.56f, 0.38f},
+     {2.16f, 2.40f, 0.702f, 0.777f, 0.00f, 2.32f, 0.50f},
+     {1.14f, 3.97f, 0.561f, 0.571f, 0.00f, 2.23f, 0.77f},
+     {2.83f, 1.32f, 0.422f, 0.450f, 0.00f, 3.17f, 0.42f}},  // [N,K]
+    {{2.41f, 0.47f, 0.611f, 0.586f, 0.72f, 2.74f, 0.21f},
+     {1.19f, 3.00f, 0.567f, 0.843f, 0.00f, 3.46f, 0.23f},
+     {3.26f, 0.01f, 0.000f, 0.707f, 0.32f, 2.69f, 0.30f},
+     {2.02f, 2.03f, 0.644f, 0.768f, 0.00f, 2.65f, 0.37f},
+     {1.47f, 2.43f, 0.500f, 0.925f, 0.00f, 2.52f, 0.47f},
+     {0.00f, 5.48f, 0.500f, 0.560f, 0.00f, 2.11f, 0.79f},
+     {3.31f, 0.36f, 0.463f, 0.487f, 0.00f, 3.21f, 0.40f}},  // [K,N]
+};
+
+// Form and split of a call with more than 16 rows.  Splits keep two steps a workgroup and 8 MiB of
+// partials, what the static scratch of fg_gemm_f16_static holds.
+int pick_tile(int M, int N, int K, bool kn, int splitk, int* split_out) {
+  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  int best = -1;
+  double best_us = 0.0;
+  for (int f = 0; f < kTileFormCount; ++f) {
+    const TileForm& t = kTileForms[f];
+    // byte offsets inside a tile are 32 bits
+    if (N % t.cols || K % t.bk || 2ull * K * std::max(t.rows, t.cols) >= (1ull << 32)) continue;
+    const TileCost& c = kTileCosts[kn][f];
+    for (int S : kSplits) {
+      if (splitk > 0 && S > 1) break;
+      if (splitk <= 0 && S > 1 && (K / t.bk < 2 * S || 4ull * S * M * N > (8u << 20))) break;
+      const int split = splitk > 0 ? splitk : S;
+      const double wgs = (double)(N / t.cols) * ceil_div(M, t.rows) * split;
+      const double q = std::ceil(wgs / kCUs), steps = std::ceil((double)(K / t.bk) / split);
+      double us = c.c + c.c2 * q + steps * std::max((double)c.t1, q * c.t2);
+      if (split > 1) us += c.s0 + c.s2 * split + c.s1 * split * ((double)M * N / 1048576.0);
+      if (best < 0 || us < best_us) {
+        best = f;
+        best_us = us;
+        *split_out = split;
+      }
     }
   }
   return best;
@@ -113,7 +182,8 @@ int finish_plan(int M, int N, int K, fg_plan_t* p) {
       }
       if (p->band != 128 && p->band != 256 && p->band != 512) return FG_ERR_UNSUPPORTED;
       if ((p->tile_n > 32 || p->tile_n % 16 != 0 || p->m_block == 32) && p->band != 128) return FG_ERR_UNSUPPORTED;
-      if (p->m_block == 32 && (p->tile_n % 16 != 0 || p->tile_n > 48)) return FG_ERR_UNSUPPORTED;
+      // (32 rows on 64 columns names the tiled kernel)
+      if (p->m_block == 32 && (p->tile_n % 16 != 0 || (p->tile_n > 48 && tile_form(M, N, K, *p) < 0))) return FG_ERR_UNSUPPORTED;
       p->unroll = p->band == 512 ? 2 : 1;
       break;
     case FG_KERNEL_KN_DOT2:
@@ -139,7 +209,9 @@ int finish_plan(int M, int N, int K, fg_plan_t* p) {
   if (p->fused < 0 || p->fused > 4) return FG_ERR_INVALID_ARG;
   if (p->splitk > 1 && p->fused >= 3 && (p->kernel != FG_KERNEL_KN_MFMA || p->splitk > kMailboxMaxSplit)) return FG_ERR_UNSUPPORTED;
   if (p->splitk > 1) {
-    if ((long long)p->grid_x * p->grid_y > kWsMaxTiles) p->fused = 0;
+    TileForm t = {0, 0, 0};
+    const long long tiles = tile_form_info(tile_form(M, N, K, *p), &t) ? (long long)(N / t.cols) * ceil_div(M, t.rows) : 0;
+    if (std::max(tiles, (long long)p->grid_x * p->grid_y) > kWsMaxTiles) p->fused = 0;
     // the in-launch completion addresses the partials with 32-bit byte offsets
     if ((unsigned long long)p->splitk * M * N * sizeof(float) > 0x7fffffffull) p->fused = 0;
     p->workspace_bytes = kWsHeaderBytes + (size_t)p->splitk * M * N * sizeof(float);
@@ -280,6 +352,32 @@ WideTile pick_wide_tile(int M, int N, int K, int splitk) {
   return best;
 }
 
+// Where the tiled kernel measured ahead of the kernels that repeat themselves per block of rows.
+bool tile_wins(int M, int N, int K, int w_layout) {
+  const size_t weights = (size_t)N * K;
+  if (M <= 16 || K < 512 || weights < ((size_t)1 << 22)) return false;  // (smaller weights were not measured)
+  if (w_layout == FG_W_KN) {
+    // Small weights stay with the 16-row kernel where its two or eight blocks of rows cost it little: a
+    // microsecond either way at 4 Mi weights (N=1024 K=4096 M=17 8.9 / 7.9 us, N=4096 K=1024 M=128
+    // 8.1 / 9.0), while M=48 takes 9.2 .. 13.5 / 7.5 .. 8.4 and M=256 15.1 / 13.1.
+    if (M <= 32) return weights > ((size_t)1 << 23);
+    return weights > ((size_t)1 << 22) || M <= 96 || M > 128;
+  }
+  if (M <= 32) {
+    // The row-load kernel reads the weights once here too.  It stays where its wide tiles land on whole
+    // CUs (N = K = 8192 M=17 24.8 / 25.6 us, N=12288 K=3072 15.1 / 15.7) unless the rows lie off
+    // 2 KB boundaries (N=4096 K=11008 20.6 / 18.8, N=6144 K=9088 29.9 / 22.7), for narrow outputs
+    // (N=2048 K=8192 10.1 / 11.4) and for small weights (N=7424 K=1408 7.1 / 8.7, N = K = 4096 9.9 /
+    // 10.6); elsewhere N=13824 K=5120 34.3 / 25.5, N = K = 5120 M=32 22.5 / 14.4.
+    const int wide = pick_wide_tile(16, N, K, 0).tile_n;
+    const bool whole_cus = wide != 0 && wide % 16 == 0 && wide <= 48 && K % 1024 == 0;
+    return N > 2048 && weights > ((size_t)1 << 24) && !whole_cus;
+  }
+  // 4 Mi weights: level or behind up to 128 rows (N = K = 2048 M=64 6.8 / 8.2 us, M=128 9.8 / 9.8, M=256
+  // 16.4 / 12.4)
+  return weights > ((size_t)1 << 22) || M > 128;
+}
+
 int make_plan(int M, int N, int K, int w_layout, int splitk, fg_plan_t* p) {
   std::memset(p, 0, sizeof(*p));
   p->stream_w = 1;
@@ -288,6 +386,23 @@ int make_plan(int M, int N, int K, int w_layout, int splitk, fg_plan_t* p) {
   // [K,N] M=1 26.4 / 25.0, M=8 26.2 / 25.2, M=16 26.5 / 25.9.  Beyond one block of 16 rows the
   // second kernel takes over.
   p->fused = M <= 16;
+  // More than 16 rows: the tiled kernel reads the weights once for up to 128 rows, the others once for
+  // every 16 or 32.  Measured against them (us, the plans below / this kernel): [K,N] N=13824 K=5120 M=17
+  // 47 / 29, M=48 85 / 32, M=256 333 / 58; N=4096 K=4096 M=64 17.6 / 13.2; [N,K] N=4096 K=11008 M=48
+  // 40 / 21, N=8192 K=8192 M=128 122 / 39, N=1024 K=16384 M=256 62 / 24.
+  if (tile_wins(M, N, K, w_layout)) {
+    const bool kn = w_layout == FG_W_KN;
+    fg_plan_t q = *p;
+    q.kernel = kn ? FG_KERNEL_KN_MFMA : FG_KERNEL_NK_MFMA_R;
+    q.tile_n = kn ? 128 : 64;
+    q.m_block = kn ? 16 : 32;
+    q.band = kn ? 0 : 128;
+    q.waves = 8, q.unroll = 1, q.fused = 1;
+    if (pick_tile(M, N, K, kn, splitk, &q.splitk) >= 0 && finish_plan(M, N, K, &q) == FG_OK) {
+      *p = q;
+      return FG_OK;
+    }
+  }
   int items = 1;
   bool row_tiles = false;   // the 16-column row-load kernel picks its own split
   bool wide_tiles = false;  // ... in its 32-column form
@@ -769,6 +884,14 @@ void set_xccs(int x) {
   if (x >= 1 && x <= 64) kXccs = x;
 }
 int xccs() { return kXccs; }
+
+int tile_form(int M, int N, int K, const fg_plan_t& p) {
+  const bool kn = p.kernel == FG_KERNEL_KN_MFMA;
+  if (!kn && (p.kernel != FG_KERNEL_NK_MFMA_R || p.m_block != 32 || p.tile_n != 64)) return -1;
+  if (!tile_wins(M, N, K, kn ? FG_W_KN : FG_W_NK)) return -1;
+  int split;
+  return pick_tile(M, N, K, kn, p.splitk < 1 ? 1 : p.splitk, &split);
+}
 
 int plan_validate_shape(int M, int N, int K, int w_layout) { return validate_shape(M, N, K, w_layout); }
 int plan_make(int M, int N, int K, int w_layout, int splitk, fg_plan_t* p) {

@@ -17,8 +17,9 @@
  *   W      fp16 weights, w_layout FG_W_KN = [K,N] row-major, FG_W_NK = [N,K] row-major
  *   C      fp16 [M,N] row-major, caller allocated
  *   K, N   multiples of 128 (the reference's only documented constraint, README.md:6-12)
- *   M      any positive value; the kernels are meant for M = 1..16 (one pass over the weights up
- *          to 32 rows with [N,K] weights, one more pass per further 32 / 16 rows)
+ *   M      any positive value: kernels of their own for M = 1..16, a tiled one beyond (one pass
+ *          over the weights for up to 128 rows; weights of less than 4 Mi elements keep the small-M
+ *          kernels, which read them once per 32 or 16 rows)
  *   arithmetic: fp16 products, fp32 accumulation, one rounding to fp16 at the end
  */
 #ifndef FASTGATE_H_
@@ -84,13 +85,17 @@ typedef struct fg_plan_t {
                        the launch; the workgroup with the last K range sums them.  If the
                        partners are not on its XCD or stay silent it computes their K ranges
                        itself (same result, slower);
+                   (Beyond 16 rows 3 and 4 complete as 1 where the tiled kernel runs.)
                    4 = as 3 with a fifth of the workgroups taking that fallback on purpose (for
                        tests).
                    0, 1, 3 and 4 sum in ascending order of S in fp32 and agree bit for bit; 2
                    sums exactly and may differ from them in the last bit                  */
   int tile_n;   /* output columns per workgroup; FG_KERNEL_NK_MFMA_R takes 16, 32, 48, 64 or,
                    with band = 128, 8 waves and no split, any divisor of N from 17 to 47  */
-  int m_block;  /* rows of A per workgroup (grid.y = ceil(M / m_block))               */
+  int m_block;  /* rows of A per workgroup (grid.y = ceil(M / m_block)).  More than 16 rows:
+                   FG_KERNEL_NK_MFMA_R with m_block 32 and tile_n 64, and FG_KERNEL_KN_MFMA, run
+                   as the tiled kernel where the library's plans use it; that picks its own tile
+                   from (M, N, K, splitk), and grid and block here are those of the named form   */
   int waves;    /* wavefronts per workgroup; they interleave over K, reduced in LDS   */
   int unroll;   /* independent 16-byte load groups in flight per lane and step        */
   int stream_w; /* 1 = weight loads carry the non-temporal hint                       */

@@ -1,0 +1,158 @@
+"""The kernel for more than 16 activation rows, through the library's plans and through forced splits and
+completions: rows at and beside the edges of its row blocks, columns and K that leave a last tile, an odd
+number of steps and fewer steps than splits.  Every output against an fp32 product on the device,
+a spread of columns against the oracle, whole numbers bit for bit."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from fastgate_amd import capi
+from helpers import ATOL, RTOL, assert_close_f16, capi_gemm, ptr, stream_ptr
+
+pytestmark = pytest.mark.gpu
+
+KN, NK = capi.FG_W_KN, capi.FG_W_NK
+EDGES = (17, 32, 33, 64, 65, 96, 97, 128, 129, 255, 256, 300)
+
+
+def _inputs(M, N, K, layout, device, whole=False, seed=0):
+    g = torch.Generator(device=device)
+    g.manual_seed(9000 + seed + M + N + K)
+    if whole:
+        A = torch.randint(-2, 3, (M, K), generator=g, device=device).half()
+        W = torch.randint(-3, 4, (K, N) if layout == KN else (N, K), generator=g, device=device).half()
+    else:
+        A = torch.randn((M, K), generator=g, device=device).half()
+        W = (torch.randn((K, N) if layout == KN else (N, K), generator=g, device=device) * 0.02).half()
+    return A, W
+
+
+def _product(A, W, layout):
+    return A.float() @ (W.float() if layout == KN else W.float().t())
+
+
+def _close(C, ref32, what):
+    assert torch.isfinite(C).all(), what
+    worst = ((C.float() - ref32).abs() - (ATOL + RTOL * ref32.abs())).max().item()
+    assert worst <= 0.0, "%s: %.4g beyond the tolerance" % (what, worst)
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("N,K", [(2048, 2176), (8320, 640), (1152, 4224), (33024, 512), (4096, 11008)])
+def test_rows_at_the_edges_of_the_row_blocks(device, layout, N, K):
+    for M in EDGES:
+        A, W = _inputs(M, N, K, layout, device)
+        out = torch.full((M + 1, N), -7.0, dtype=torch.half, device=device)  # a row behind C that stays as it is
+        p = capi_gemm(A, W, out[:M], layout)
+        what = "M=%d N=%d K=%d layout=%d %s" % (M, N, K, layout, p.as_dict())
+        _close(out[:M], _product(A, W, layout), what)
+        assert bool((out[M] == -7.0).all()), what
+        if M in (33, 129):
+            cols = torch.tensor(sorted({0, 1, 63, 64, 127, N // 2 + 5, N - 65, N - 1}), device=device)
+            sub = (W[:, cols].t() if layout == KN else W[cols]).contiguous().cpu().numpy()
+            ref, _ = oracle.gemm_f16(A.cpu().numpy(), sub, oracle.W_NK)
+            assert_close_f16(out[:M][:, cols].cpu().numpy(), ref, what)
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("M", [33, 96, 130])
+def test_splits_and_completions_agree(device, layout, M):
+    # whole numbers: every split and completion gives the exact sum; 40 splits leave workgroups without a step
+    N, K = 1920, 2304
+    A, W = _inputs(M, N, K, layout, device, whole=True)
+    exact = _product(A, W, layout).half()
+    for splitk in (1, 2, 5, 17, 40):
+        for fused in ((0, 1, 2, 3) if layout == KN else (0, 1, 2)):
+            p = capi.plan(M, N, K, layout, splitk)
+            if fused == 2 and (splitk > 31 or M * N > 262144):
+                continue
+            if fused == 3 and splitk > 32:
+                continue
+            p.fused = fused
+            C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
+            for _ in range(2):  # the second call finds the header as the first left it
+                capi_gemm(A, W, C, layout, plan=p)
+                assert torch.equal(C, exact), (splitk, fused)
+    # two passes and the counters add the same partials in the same order
+    A, W = _inputs(M, N, K, layout, device, seed=1)
+    got = []
+    for fused in (0, 1):
+        p = capi.plan(M, N, K, layout, 3)
+        p.fused = fused
+        got.append(torch.empty((M, N), dtype=torch.half, device=device))
+        capi_gemm(A, W, got[-1], layout, plan=p)
+    assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("splitk", [1, 3])
+def test_accumulate_bias_activation_and_pitch(device, layout, splitk):
+    M, N, K = 70, 1664, 2688
+    L = capi.lib()
+    A, W = _inputs(M, N, K, layout, device)
+    ref = _product(A, W, layout)
+    C0 = torch.randn((M, N), device=device).half()
+    C = C0.clone()
+    capi_gemm(A, W, C, layout, accumulate=True, splitk=splitk)
+    _close(C, ref + C0.float(), "accumulate")
+    bias = torch.randn(N, device=device).half()
+    ws = torch.zeros(capi.plan(M, N, K, layout, splitk).workspace_bytes + 16, dtype=torch.uint8, device=device)
+    st = L.fg_gemm_f16_bias_act(ptr(A), ptr(W), ptr(bias), 4, ptr(C), M, N, K, layout, splitk, None, ptr(ws),
+                                ws.numel(), stream_ptr())
+    assert st == capi.FG_OK
+    _close(C, torch.nn.functional.silu(ref + bias.float()), "bias and silu")
+    if layout == KN:
+        dense = torch.empty_like(C)
+        capi_gemm(A, W, dense, layout, splitk=splitk)
+        wide = torch.full((K, N + 136), float("nan"), dtype=torch.half, device=device)
+        wide[:, :N] = W
+        st = L.fg_gemm_f16_pitched(ptr(A), ptr(wide), ptr(C), M, N, K, N + 136, 0, splitk, ptr(ws), ws.numel(),
+                                   stream_ptr())
+        assert st == capi.FG_OK and torch.equal(C, dense)
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+def test_infinities_and_nan_stay_in_their_rows(device, layout):
+    M, N, K = 50, 2048, 2304
+    A, W = _inputs(M, N, K, layout, device)
+    A[3, 100] = float("inf")
+    A[49, K - 1] = float("nan")
+    C = torch.empty((M, N), dtype=torch.half, device=device)
+    capi_gemm(A, W, C, layout)
+    ref = _product(A, W, layout)
+    col = (W[100] if layout == KN else W[:, 100]) != 0
+    assert bool(torch.isinf(C[3][col]).all()) and bool((torch.sign(C[3][col].float()) == torch.sign(ref[3][col])).all())
+    assert bool(torch.isnan(C[49]).all())
+    rest = [m for m in range(M) if m not in (3, 49)]
+    _close(C[rest], ref[rest], "rows beside them")
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+def test_replayed_graph_gives_the_eager_result(device, layout):
+    M, N, K = 48, 2048, 4352
+    A, W = _inputs(M, N, K, layout, device)
+    C, want = (torch.empty((M, N), dtype=torch.half, device=device) for _ in range(2))
+    p = capi.plan(M, N, K, layout)
+    assert p.splitk > 1
+    ws = torch.zeros(p.workspace_bytes, dtype=torch.uint8, device=device)
+
+    def call(out):
+        st = capi.lib().fg_gemm_f16_planned(ptr(A), ptr(W), ptr(out), M, N, K, layout, 0, ctypes.byref(p), ptr(ws),
+                                            ws.numel(), stream_ptr())
+        capi.check(st, "fg_gemm_f16_planned")
+
+    call(C)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(C)
+    for i in range(4):
+        A.copy_(torch.randn((M, K), device=device).half())
+        C.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        call(want)
+        assert torch.equal(C, want), i
