@@ -562,6 +562,133 @@ __global__ __launch_bounds__(512) void w4a16_r_kernel(const uint8_t* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------
+// w4a16, two to four activation rows: all activations of the workgroup in LDS, the weights from memory
+// straight into the MFMA operand.  A 4-row activation panel is 8 bytes a k, so all of it fits
+// LDS up to KC = 16384 k; every wave has its whole share of the tile's weight rows in flight (loads of
+// 16 rows x 64 bytes) while the panel is staged, and nothing but the decode stands between a weight's
+// arrival and its product: no LDS round trip for the weights and one memory latency a call.  Launched
+// with K <= KC.  What bounds it: launch and the two streams, weights from memory and as many or
+// twice as many panel bytes from L2 (M=4 N=4096 K=14336, 29 MB: 11.5 us, 2.6 TB/s, a plain read 5.7;
+// N=14336 K=4096 9.3); the row-load kernel above takes 13.0 and 13.2, with five operations more a word
+// and both operands through LDS.
+//  * Lane (j, g) loads 16 bytes = 32 k of row j: four words of eight nibbles.  The even nibbles of
+//    two words make one MFMA operand (nibbles 0,4,2,6 of each), the odd ones a second: masked in
+//    place they are fp16 subnormals, n 2^-24 and n 2^-20, exactly, so five integer operations
+//    decode eight weights and two accumulators keep the two powers of two apart.
+//  * The panel lies in LDS in that order: 16-byte pieces [load][word pair][even, odd][g][row], so one
+//    operand read of a wave covers 256 contiguous bytes (the lanes of rows 4..15 repeat rows 0..3).
+//  * The row sums for the zero point are taken while the panel is staged.
+// ---------------------------------------------------------------------------------------
+template <int KC, int CB, int NW>
+__global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restrict__ Wq, const half_t* __restrict__ X,
+                                                      const half_t* __restrict__ scale, float scalar_scale,
+                                                      float zero_point, half_t* __restrict__ Y, int M, int N, int K) {
+  constexpr int LOADS = KC / 128 / NW;     // weight loads a wave
+  constexpr int GROUPS = KC / 16 / (16 * NW);    // 16-k groups of its activation row a thread
+  __shared__ u32x4 panel[KC / 2];          // 4 rows x KC halves
+  __shared__ float red[NW][CB][2][64];
+  __shared__ float xred[NW][4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (16 * CB);
+  const size_t rowb = (size_t)K >> 1;
+  // scale of the output this thread writes at the end, fetched ahead of the weight stream
+  const uint32_t scale_raw = scale_fetch(scale, n0 + (tid >> 6) * 16 + (tid & 15), tid < 64 * CB);
+  constexpr int kNonTemporal = 2;
+  const __amdgpu_buffer_rsrc_t wrs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(Wq + (size_t)n0 * rowb), 0, (int)(16 * CB * rowb), 0x00020000);
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(X), 0, M * K * 2, 0x00020000);
+  constexpr int kBeyond = 0x7ffffff0;      // past both descriptors: the load returns zeros
+  const int xm = tid & 3, xq = tid >> 2;   // this thread's activation row and first group
+  const half2_t ones = {static_cast<half_t>(1.f), static_cast<half_t>(1.f)};
+  float4_t even[CB], odd[CB];
+#pragma unroll
+  for (int b = 0; b < CB; ++b) even[b] = odd[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+  float xsum = 0.f;
+  auto load_of = [&](int t) { return wave + NW * t; };
+  const int loads = K >> 7;
+  u32x4 x0[GROUPS], x1[GROUPS], w[CB][LOADS];
+  // activations first: loads return in order, and the panel must not wait for the weights
+#pragma unroll
+  for (int i = 0; i < GROUPS; ++i) {
+    const int q = xq + 16 * NW * i;
+    const int off = (q * 16 < K && xm < M) ? (xm * K + q * 16) * 2 : kBeyond;
+    x0[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+    x1[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 16, 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < LOADS; ++t) {
+    const int l = load_of(t);
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int off = l < loads ? (16 * b + j) * (int)rowb + l * 64 + g * 16 : kBeyond;
+      w[b][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, 0, kNonTemporal));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < GROUPS; ++i) {
+    const int q = xq + 16 * NW * i;
+    const u32x4 a = x0[i], b = x1[i];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      xsum = __builtin_amdgcn_fdot2(as_half2(a[c]), ones, xsum, false);
+      xsum = __builtin_amdgcn_fdot2(as_half2(b[c]), ones, xsum, false);
+    }
+    constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;
+    u32x4* at = panel + (q >> 3) * 64 + (q & 1) * 32 + ((q >> 1) & 3) * 4 + xm;
+    at[0] = u32x4{__builtin_amdgcn_perm(a.z, a.x, kLow), __builtin_amdgcn_perm(a.w, a.y, kLow),
+                  __builtin_amdgcn_perm(b.z, b.x, kLow), __builtin_amdgcn_perm(b.w, b.y, kLow)};
+    at[16] = u32x4{__builtin_amdgcn_perm(a.z, a.x, kHigh), __builtin_amdgcn_perm(a.w, a.y, kHigh),
+                   __builtin_amdgcn_perm(b.z, b.x, kHigh), __builtin_amdgcn_perm(b.w, b.y, kHigh)};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < LOADS; ++t) {        // (past the end of K: zero weights on a zero panel)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const u32x4* at = panel + (load_of(t) * 2 + p) * 32 + g * 4 + (j & 3);
+      const u32x4 xe = at[0], xo = at[16];
+#pragma unroll
+      for (int b = 0; b < CB; ++b) {
+        const uint32_t u = w[b][t][2 * p], v = w[b][t][2 * p + 1], u8 = u >> 8, v8 = v >> 8;
+        const u32x4 we = {u & 0x000F000Fu, u8 & 0x000F000Fu, v & 0x000F000Fu, v8 & 0x000F000Fu};  // 0,4 2,6 of both
+        const u32x4 wo = {u & 0x00F000F0u, u8 & 0x00F000F0u, v & 0x00F000F0u, v8 & 0x00F000F0u};  // 1,5 3,7
+        even[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xe), as_half8(we), even[b], 0, 0, 0);
+        odd[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xo), as_half8(wo), odd[b], 0, 0, 0);
+      }
+    }
+  }
+  // lanes 0..15 hold rows 0..3 of column j in registers 0..3; lanes of one activation row sit 4 apart
+#pragma unroll
+  for (int d = 4; d < 64; d <<= 1) xsum += __shfl_xor(xsum, d);
+  if (lane < 4) xred[wave][lane] = xsum;
+  if (lane < 16) {
+#pragma unroll
+    for (int b = 0; b < CB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        red[wave][b][0][r * 16 + j] = even[b][r];
+        red[wave][b][1][r * 16 + j] = odd[b][r];
+      }
+  }
+  __syncthreads();
+  if (tid < 64 * CB) {
+    const int b = tid >> 6, e = tid & 63, m = e >> 4, n = n0 + 16 * b + (e & 15);
+    if (m < M) {
+      const float se = lds_sum<NW>(&red[0][b][0][e], 128 * CB, NW), so = lds_sum<NW>(&red[0][b][1][e], 128 * CB, NW);
+      const float xs = lds_sum<NW>(&xred[0][m], 4, NW);
+      float v = (se * 16777216.f + so * 1048576.f) - zero_point * xs;
+      if (not_finite(xs)) v = elementwise_dot<4>(Wq + (size_t)n * rowb, X + (size_t)m * K, K, zero_point);
+      Y[(size_t)m * N + n] = static_cast<half_t>(v * (scalar_scale * scale_value(scale_raw)));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Host launchers.  The integer-dot kernel: rows per workgroup 8 when that still yields >= 512
 // workgroups, else 4; waves per workgroup as many (<= 4) as the row has 1 KB pieces.
 // ---------------------------------------------------------------------------------------
@@ -683,6 +810,39 @@ bool launch_w8a16(const W8A16Args& a, hipStream_t s) {
   return true;
 }
 
+// Panel kernel (w4a16_x_kernel): where it measured ahead, us, the kernel it replaces / this one.
+//  * three and four rows, K up to 16384 (one pass): M=4 N=14336 K=5120 18.2 / 12.5, N=28672 K=2304 18.0 /
+//    12.0, N=12288 K=3072 10.5 / 7.6, N = K = 8192 12.7 / 11.2, N=4096 K=4096 6.0 / 4.7, K=14336 13.0 / 11.5;
+//    not with a second pass (N=4096 K=20480 15.4 / 19.3).  Narrow outputs leave its tiles on half the
+//    CUs: four rows still gain beyond 1024 columns (N=2048 K=8192 7.5 / 6.5), three are level (N = K = 2048 3.8 /
+//    3.8), N=1024 K=4096 M=3 4.0 / 4.2, K=16384 M=4 7.6 / 11.7.
+//  * two rows: the lanes-over-x kernel reads half the activations it does at four, so only for K up to
+//    4096 (N = K = 4096 4.9 / 4.4, N=28672 K=2304 13.9 / 11.3, N=12288 K=3072 7.5 / 6.8; N = K = 5120 6.4 / 7.7).
+static bool w4_panel(const W8A16Args& a) {
+  if (a.K > 16384) return false;
+  if (a.M == 2) return a.N > 2048 && a.K <= 4096;
+  return a.N > 2048 || (a.M == 4 && a.N > 1024 && a.K <= 8192);
+}
+static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
+#define FG_W4_X(KC, CB, NW)                                                                                     \
+  hipLaunchKernelGGL((w4a16_x_kernel<KC, CB, NW>), dim3(a.N / (16 * CB)), dim3(64 * NW), 0, s,                  \
+                     static_cast<const uint8_t*>(a.Wq), static_cast<const half_t*>(a.x),                       \
+                     static_cast<const half_t*>(a.scale), a.scalar_scale, a.zero_point, static_cast<half_t*>(a.y), \
+                     a.M, a.N, a.K)
+  // 32 columns a workgroup stage the panel half as often, where N / 32 workgroups fill the CUs evenly
+  // (M=4 N=14336 K=4096 10.7 / 9.3; N=12288 K=3072, 384 workgroups, 7.6 / 8.6 the other way).  KC: the
+  // smallest that holds K; sixteen waves share the largest panels (K=14336 11.9 / 11.5 with eight).
+  const int t32 = a.N / 32;
+  const bool wide = t32 >= 224 && 8 * t32 >= 7 * ((t32 + 255) / 256 * 256);
+  if (a.K <= 2048) { if (wide) FG_W4_X(2048, 2, 8); else FG_W4_X(2048, 1, 8); }
+  else if (a.K <= 4096) { if (wide) FG_W4_X(4096, 2, 8); else FG_W4_X(4096, 1, 8); }
+  else if (a.K <= 6144) { if (wide) FG_W4_X(6144, 2, 8); else FG_W4_X(6144, 1, 8); }
+  else if (a.K <= 8192) { if (wide) FG_W4_X(8192, 2, 8); else FG_W4_X(8192, 1, 8); }
+  else if (a.K <= 12288) FG_W4_X(12288, 1, 16);
+  else FG_W4_X(16384, 1, 16);
+#undef FG_W4_X
+}
+
 bool launch_w4a16(const W8A16Args& a, hipStream_t s) {
   auto* Wq = static_cast<const uint8_t*>(a.Wq);
   auto* X = static_cast<const half_t*>(a.x);
@@ -691,6 +851,8 @@ bool launch_w4a16(const W8A16Args& a, hipStream_t s) {
   if (a.M < 1 || a.M > 4) return false;
   if (a.M == 1) {
     launch_wq_m1<4, 1>(a, s);
+  } else if (w4_panel(a)) {
+    launch_w4_panel(a, s);
   } else if (a.M == 2) {
     launch_wq_m1<4, 2>(a, s);
   } else if (a.N <= 2048) {

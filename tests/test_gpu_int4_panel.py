@@ -1,0 +1,70 @@
+"""int4 weights against two to four activation rows held in LDS as one panel: K at and beside the panel
+sizes (and beyond the largest, where the row-load kernel takes over), one and two column blocks a
+workgroup.  Single weights picked out come back exactly; sums are held to the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from fastgate_amd import capi
+from helpers import assert_close_f16, gen, normal, ptr, stream_ptr
+
+pytestmark = pytest.mark.gpu
+
+PANELS = (2048, 4096, 6144, 8192, 12288, 16384)
+KS = (128, *[k + d for k in PANELS for d in (-128, 0, 128)])
+
+
+def _run(Wd, x, scale, scalar_scale, zp, device):
+    M, K = x.shape
+    N = Wd.shape[0]
+    y = torch.full((M + 1, N), 5.0, dtype=torch.half, device=device)  # a row behind the result stays as it is
+    xd = x.to(device)
+    capi.check(capi.lib().fg_gemv_w4a16(ptr(Wd), ptr(xd), ptr(scale), scalar_scale, zp, ptr(y), M, N, K, stream_ptr()),
+               "fg_gemv_w4a16")
+    torch.cuda.synchronize()
+    assert bool((y[M] == 5.0).all())
+    return y[:M].cpu().numpy()
+
+
+@pytest.mark.parametrize("K", KS)
+@pytest.mark.parametrize("N", [2176, 7168])  # 16 columns a workgroup; 32 (224 workgroups)
+def test_panel_sizes(device, N, K):
+    g = torch.Generator(device=device)
+    g.manual_seed(9300 + N + K)
+    Wd = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=device)
+    W = Wd.cpu().numpy()
+    scale = (torch.rand(N, generator=g, device=device) * 0.009 + 0.001).half()
+    cols = np.array(sorted({0, 1, 15, 16, 31, 32, N // 2 + 7, N - 33, N - 16, N - 1}))
+    for M in (2, 3, 4):
+        x = normal((M, K), gen(9400 + M + K))
+        got = _run(Wd, x, scale, 0.5, 7.5, device)
+        ref, _ = oracle.gemv_w4a16(W[cols], x.numpy(), scale.cpu().numpy()[cols], 0.5, 7.5)
+        assert_close_f16(got[:, cols], ref, "M=%d N=%d K=%d" % (M, N, K))
+        # x = e_k: the output is the weight, at positions over a 128-k load and at the end of K
+        for k in sorted({0, 1, 7, 8, 30, 63, 64, 127, K // 2 + 21, K - 97, K - 2, K - M}):
+            if k < 0 or k + M > K:
+                continue
+            x = torch.zeros((M, K), dtype=torch.half)
+            for m in range(M):
+                x[m, k + m] = 1.0
+            got = _run(Wd, x, None, 1.0, 8.0, device)
+            for m in range(M):
+                b = W[:, (k + m) // 2]
+                want = (b >> 4 if (k + m) % 2 else b & 15).astype(np.float32) - 8.0
+                assert (got[m].astype(np.float32) == want).all(), (M, K, k, m)
+
+
+@pytest.mark.parametrize("N,K", [(2176, 4096), (7168, 6272)])
+def test_broken_rows_stay_alone(device, N, K):
+    g = gen(9500 + K)
+    Wd = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8).to(device)
+    x = normal((4, K), g)
+    x[1, 5] = float("inf")
+    x[3, K - 1] = float("nan")
+    got = _run(Wd, x, None, 1.0, 8.0, device)
+    ref, _ = oracle.gemv_w4a16(Wd.cpu().numpy()[:64], x.numpy()[[0, 2]], None, 1.0, 8.0)
+    assert_close_f16(got[[0, 2]][:, :64], ref, "finite rows")
+    w = (Wd[:, 2] >> 4).cpu().numpy().astype(np.float32) - 8.0  # k = 5: the high nibble of byte 2
+    assert (np.isnan(got[1]) == (w == 0)).all() and (np.sign(got[1][w != 0]) == np.sign(w[w != 0])).all()
+    assert np.isinf(got[1][w != 0]).all() and np.isnan(got[3]).all()
