@@ -275,6 +275,70 @@ __global__ __launch_bounds__(256) void i8i8_kernel(const int8_t* __restrict__ Wq
   }
 }
 
+// Two to eight activation rows: as w4a16_x_kernel below, the activation panel in LDS and the weights from
+// memory straight into the operand of v_mfma_i32_16x16x64_i8 (16 bytes = 16 k of row j a lane), every
+// load of a wave's share in flight before the panel is staged.  XR = rows of the panel, 4 or 8; its
+// 16-byte pieces lie as [load][g][row].  Integer sums: exact in any order.  Launched with K <= KC.
+template <int XR, int KC, int NW>
+__global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restrict__ Wq, const int8_t* __restrict__ Xq,
+                                                         int32_t* __restrict__ out, int M, int N, int K) {
+  typedef int int4_v __attribute__((ext_vector_type(4)));
+  constexpr int NT = 64 * NW;
+  constexpr int LOADS = KC / 64 / NW;         // weight loads a wave
+  constexpr int PIECES = XR * KC / 16 / NT;   // pieces of the panel a thread
+  static_assert(KC % (64 * NW) == 0 && XR * KC % (16 * NT) == 0, "whole loads and pieces");
+  __shared__ u32x4 panel[XR * KC / 16];
+  __shared__ int red[NW][XR * 16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  constexpr int kNonTemporal = 2;
+  const __amdgpu_buffer_rsrc_t wrs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Wq + (size_t)n0 * K), 0, 16 * K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Xq), 0, M * K, 0x00020000);
+  constexpr int kBeyond = 0x7ffffff0;         // past both descriptors: the load returns zeros
+  const int xm = tid % XR, xq = tid / XR;     // this thread's activation row and first 16-k piece of it
+  const int loads = K >> 6;
+  u32x4 x[PIECES], w[LOADS];
+  // activations first: loads return in order, and the panel must not wait for the weights
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int q = xq + NT / XR * i;
+    const int off = (q * 16 < K && xm < M) ? xm * K + q * 16 : kBeyond;
+    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < LOADS; ++t) {
+    const int l = wave + NW * t;
+    const int off = l < loads ? j * K + l * 64 + g * 16 : kBeyond;
+    w[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, 0, kNonTemporal));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) panel[(xq + NT / XR * i) * XR + xm] = x[i];
+  __syncthreads();
+  int4_v acc = {0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < LOADS; ++t)             // (past the end of K: zero weights on a zero panel)
+    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+        __builtin_bit_cast(int4_v, panel[((wave + NW * t) * 4 + g) * XR + j % XR]), __builtin_bit_cast(int4_v, w[t]),
+        acc, 0, 0, 0);
+  // acc[r]: row 4g + r, column j
+  if (4 * g < XR) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][(4 * g + r) * 16 + j] = acc[r];
+  }
+  __syncthreads();
+  if (tid < XR * 16) {
+    int sum = 0;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) sum += red[v][tid];
+    if ((tid >> 4) < M) out[(size_t)(tid >> 4) * N + n0 + (tid & 15)] = sum;
+  }
+}
+
 __global__ __launch_bounds__(256) void dequant_i32_f16_kernel(const int32_t* __restrict__ acc,
                                                               const half_t* __restrict__ scale,
                                                               float x_scale, half_t* __restrict__ y,
@@ -885,13 +949,52 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
   }
 }
 
+// Panel kernel (i8i8_x_kernel): where it measured ahead, us, the v_dot4 kernel / this one.
+//  * five to eight rows, which cost the v_dot4 kernel a register tile per row: M=8 N=14336 K=4096 22.9 / 16.6,
+//    K=5120 24.5 / 20.7; N = K = 8192 19.1 / 16.0, N = K = 4096 8.8 / 5.9; N=4096 K=14336 16.7 / 14.9.  Not
+//    narrow outputs with long rows (N=2048 K=8192 7.7 / 8.2, K=4096 5.9 / 5.1; N=1024 K=4096 4.7 / 5.0), and
+//    not tiles that leave a third of the CUs' second round idle (N = K = 5120, 320 tiles, M=5 10.5 / 10.6).
+//  * two to four rows: short rows (M=4 N=7168 K=2048 6.1 / 5.1, N=11008 K=1024 6.2 / 4.6, N = K = 2048
+//    3.9 / 3.5), and three and four where the tiles fill the CUs exactly (N = K = 4096 6.8 / 5.7, N=4096
+//    K=6144 7.7 / 6.9, N=16384 K=4096 16.4 / 15.6; N=14336 K=4096 14.6 / 15.2).  Elsewhere 1 KB of a row a
+//    load beats 16 rows x 64 bytes (N = K = 8192 13.6 / 14.4, N = K = 5120 8.2 / 10.3).
+static bool i8_panel(int M, int N, int K) {
+  if (M < 2 || N < 2048 || K > 16384) return false;
+  const int tiles = N / 16;
+  if (M >= 5) {
+    const bool even = 10 * tiles >= 7 * ((tiles + 255) / 256 * 256);
+    return K <= 4096 || (N > 2048 && even);
+  }
+  return K <= 2048 || (M >= 3 && K <= 6144 && (tiles == 256 || tiles == 512 || tiles == 1024) && (K <= 4096 || tiles == 256));
+}
+
 bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N, int K,
                      hipStream_t s) {
-  if (M == 1) i8i8_go<1>(Wq, xq, acc, M, N, K, s);
-  else if (M == 2) i8i8_go<2>(Wq, xq, acc, M, N, K, s);
-  else if (M <= 4) i8i8_go<4>(Wq, xq, acc, M, N, K, s);
-  else if (M <= 8) i8i8_go<8>(Wq, xq, acc, M, N, K, s);
-  else return false;
+  if (M < 1 || M > 8) return false;
+  if (i8_panel(M, N, K)) {
+    auto* W = static_cast<const int8_t*>(Wq);
+    auto* X = static_cast<const int8_t*>(xq);
+#define FG_I8_X(XR, KC, NW) \
+  hipLaunchKernelGGL((i8i8_x_kernel<XR, KC, NW>), dim3(N / 16), dim3(64 * NW), 0, s, W, X, acc, M, N, K)
+#define FG_I8_X_KC(XR)                            \
+  if (K <= 2048) FG_I8_X(XR, 2048, 8);             \
+  else if (K <= 4096) FG_I8_X(XR, 4096, 8);        \
+  else if (K <= 6144) FG_I8_X(XR, 6144, 8);        \
+  else if (K <= 8192) FG_I8_X(XR, 8192, 8);        \
+  else if (K <= 12288) FG_I8_X(XR, 12288, 16);     \
+  else FG_I8_X(XR, 16384, 16)
+    if (M <= 4) { FG_I8_X_KC(4); } else { FG_I8_X_KC(8); }
+#undef FG_I8_X_KC
+#undef FG_I8_X
+  } else if (M == 1) {
+    i8i8_go<1>(Wq, xq, acc, M, N, K, s);
+  } else if (M == 2) {
+    i8i8_go<2>(Wq, xq, acc, M, N, K, s);
+  } else if (M <= 4) {
+    i8i8_go<4>(Wq, xq, acc, M, N, K, s);
+  } else {
+    i8i8_go<8>(Wq, xq, acc, M, N, K, s);
+  }
   return true;
 }
 

@@ -1,0 +1,27 @@
+"""int8 x int8 products through the kernel that holds two to eight activation rows in LDS as one panel: K at
+and beside the panel sizes, both panel heights, whole int8 range, exact to the bit; nothing is written
+behind the result."""
+import pytest
+import torch
+
+from fastgate_amd import capi
+from helpers import ptr, stream_ptr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N", [2048, 2304, 4096])
+@pytest.mark.parametrize("K", (128, *[k + d for k in (2048, 4096, 6144, 8192, 12288, 16384) for d in (-128, 0, 128)]))
+def test_panel_sizes_are_exact(device, N, K):
+    g = torch.Generator(device=device)
+    g.manual_seed(9600 + N + K)
+    W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)
+    W64 = W.double().t()
+    for M in range(2, 9):
+        x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=device)
+        acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
+        st = capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr())
+        assert st == capi.FG_OK
+        want = (x.double() @ W64).round().int()  # below 2^53: exact
+        assert torch.equal(acc[:M], want), (M, N, K)
+        assert bool((acc[M] == -3).all())
