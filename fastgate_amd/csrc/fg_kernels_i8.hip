@@ -753,8 +753,8 @@ __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restr
 }
 
 // ---------------------------------------------------------------------------------------
-// Host launchers.  The integer-dot kernel: rows per workgroup 8 when that still yields >= 512
-// workgroups, else 4; waves per workgroup as many (<= 4) as the row has 1 KB pieces.
+// Host launchers.  The integer-dot kernel, beyond what i8i8_go says of two to four rows: rows per workgroup
+// 8 when that still yields >= 512 workgroups, else 4; waves as many (<= 4) as the row has 1 KB pieces.
 // ---------------------------------------------------------------------------------------
 static int i8_waves(int K) {
   const int pieces = (K / 16 + 63) / 64;
@@ -937,6 +937,21 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
                     hipStream_t s) {
   auto* W = static_cast<const int8_t*>(Wq);
   auto* X = static_cast<const int8_t*>(xq);
+  // Two to four rows: four weight rows a workgroup, one 1 KB piece of each in flight a wave, and three or
+  // four waves, whichever leaves fewer of the last step's waves without a piece -- except whole
+  // multiples of 8 KB rows, which two pieces of eight rows on four waves divide evenly (M=4, us, eight rows
+  // and two pieces / this: N = K = 5120 8.3 / 7.5, N=14336 K=4096 14.3 / 12.3, N=12288 K=3072 11.0 / 9.0,
+  // N=3072 K=9088 8.5 / 7.7, N=4096 K=11008 12.1 / 10.9, but N = K = 8192 13.6 / 13.9).  Narrow outputs keep two
+  // pieces in flight, their workgroups do not fill the chip (N=2048 K=14336 M=4 7.9 / 8.5), and the
+  // longest rows are level (N=4096 K=14336 M=4 12.8 / 13.0).
+  if (MB == 2 || MB == 4) {
+    const int pieces = (K / 16 + 63) / 64;
+    if (N > 2048 && K <= 12288 && K % 8192 != 0) {
+      const int waves = pieces <= 4 ? pieces : ((pieces + 2) / 3 * 3 < (pieces + 3) / 4 * 4 ? 3 : 4);
+      hipLaunchKernelGGL((i8i8_kernel<MB, 4, 1>), dim3(N / 4), dim3(64 * waves), 0, s, W, X, acc, M, N, K);
+      return;
+    }
+  }
   const dim3 block(64 * i8_waves(K));
   if (MB == 1) {
     hipLaunchKernelGGL((i8i8_kernel<1, 4, 1>), dim3(N / 4), block, 0, s, W, X, acc, M, N, K);

@@ -25,3 +25,17 @@ def test_panel_sizes_are_exact(device, N, K):
         want = (x.double() @ W64).round().int()  # below 2^53: exact
         assert torch.equal(acc[:M], want), (M, N, K)
         assert bool((acc[M] == -3).all())
+
+
+@pytest.mark.parametrize("N,K", [(2176, 2304), (2176, 4992), (3072, 6144), (4224, 9088), (5120, 5120), (2176, 8192)])
+def test_few_rows_beside_the_panel_are_exact(device, N, K):
+    # the v_dot4 kernel on three or four waves: K that gives every wave a piece, and K that does not
+    g = torch.Generator(device=device)
+    g.manual_seed(9700 + N + K)
+    W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)
+    for M in (2, 3, 4):
+        x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=device)
+        acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
+        assert capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr()) == capi.FG_OK
+        assert torch.equal(acc[:M], (x.double() @ W.double().t()).round().int()), (M, N, K)
+        assert bool((acc[M] == -3).all())
