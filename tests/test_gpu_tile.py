@@ -156,3 +156,22 @@ def test_replayed_graph_gives_the_eager_result(device, layout):
         torch.cuda.synchronize()
         call(want)
         assert torch.equal(C, want), i
+
+
+@pytest.mark.parametrize("M", [33, 65])
+def test_nk_rows_of_16_mi_elements(device, M):
+    # a row of W is 32 MiB, a tile's rows together more than 2 GiB; -1, 0 and 1 keep every partial sum a
+    # whole number below 2^24, exact in fp32 in any order
+    N, K = 128, 1 << 24
+    g = torch.Generator(device=device)
+    g.manual_seed(9100 + M)
+    A = torch.randint(-1, 2, (M, K), generator=g, dtype=torch.int8, device=device).half()
+    W = torch.randint(-1, 2, (N, K), generator=g, dtype=torch.int8, device=device).half()
+    want = torch.zeros((M, N), device=device)
+    for k in range(0, K, 1 << 20):
+        want += A[:, k:k + (1 << 20)].float() @ W[:, k:k + (1 << 20)].float().t()
+    C = torch.full((M + 1, N), -7.0, dtype=torch.half, device=device)
+    for splitk in (0, 1):
+        capi_gemm(A, W, C[:M], NK, splitk=splitk)
+        assert torch.equal(C[:M], want.half()), splitk
+        assert bool((C[M] == -7.0).all())

@@ -313,6 +313,20 @@ def test_compute_entry_points_validate_before_touching_the_device():
     assert L.fg_gemm_f16_planned(one, one, one, 1, 256, 256, NK, 0, ctypes.byref(bad), None, 0, None) == capi.FG_ERR_UNSUPPORTED
 
 
+# A call that passes every check of the host code ends in a failed launch where there is no device.  The
+# pointers are made up, so nothing of this may run where a launch would succeed.
+without_device = pytest.mark.skipif(Path("/dev/kfd").exists(), reason="the call would be launched")
+
+
+@without_device
+@pytest.mark.parametrize("M,N,K", [(33, 128, 1 << 24), (64, 1024, 1 << 24), (48, 256, (1 << 24) + 128),
+                                   (300, 128, 1 << 24), (33, 128, (1 << 25) - 128), (33, 128, 1 << 25),
+                                   (17, 4096, 1 << 24)])
+def test_nk_rows_of_16_mi_elements_reach_a_kernel(M, N, K):
+    one = ctypes.c_void_p(16)
+    assert capi.lib().fg_gemm_f16(one, one, one, M, N, K, NK, 0, 1, None, 0, None) == capi.FG_ERR_LAUNCH
+
+
 # ---- pybind11 surface ---------------------------------------------------------------------------
 REFERENCE_NAMES = {
     # backend/cuda/hk/edgemm.h:4-14
