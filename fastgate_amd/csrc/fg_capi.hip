@@ -99,6 +99,15 @@ int run_gemm(const void* A, const void* W, void* C, int M, int N, int K, int acc
   return FG_OK;
 }
 
+// The plan of a call that leaves it to the library.  The library's own choice of a split (splitk 0) needs
+// a workspace; where the caller did not bring one, or too small a one, the call runs unsplit (slower
+// where the grid then leaves CUs idle) instead of failing.
+int plan_for_workspace(int M, int N, int K, int w_layout, int splitk, const void* ws, size_t ws_bytes, fg_plan_t* p) {
+  const int st = fg_plan(M, N, K, w_layout, splitk, p);
+  if (st != FG_OK || splitk != 0 || p->splitk == 1 || (ws != nullptr && ws_bytes >= p->workspace_bytes)) return st;
+  return fg_plan(M, N, K, w_layout, 1, p);
+}
+
 // Device address of `scratch` on the current device, resolved once per device (with that device
 // current) and kept.  The first resolution also clears the counter header with a fill kernel on
 // `s`; after that every call leaves the counters at zero by itself.  Returns null on failure.
@@ -221,14 +230,8 @@ int fg_gemm_f16(const void* A, const void* W, void* C, int M, int N, int K, int 
   if (A == nullptr || W == nullptr || C == nullptr) return FG_ERR_INVALID_ARG;
   fg::read_compute_units();
   fg_plan_t p;
-  int st = fg_plan(M, N, K, w_layout, splitk, &p);
+  const int st = fg::plan_for_workspace(M, N, K, w_layout, splitk, ws, ws_bytes, &p);
   if (st != FG_OK) return st;
-  if (splitk == 0 && p.splitk > 1 && (ws == nullptr || ws_bytes < p.workspace_bytes)) {
-    // the library's own choice of a split needs a workspace the caller did not bring: run
-    // unsplit (slower where the grid then leaves CUs idle) instead of failing
-    st = fg_plan(M, N, K, w_layout, 1, &p);
-    if (st != FG_OK) return st;
-  }
   return fg::run_gemm(A, W, C, M, N, K, accumulate, p, ws, ws_bytes,
                       static_cast<hipStream_t>(stream));
 }
@@ -256,12 +259,8 @@ int fg_gemm_f16_pitched(const void* A, const void* W, void* C, int M, int N, int
   if (ldw < N || ldw % 8 != 0) return FG_ERR_INVALID_ARG;
   fg::read_compute_units();
   fg_plan_t p;
-  int st = fg_plan(M, N, K, FG_W_KN, splitk, &p);
+  const int st = fg::plan_for_workspace(M, N, K, FG_W_KN, splitk, ws, ws_bytes, &p);
   if (st != FG_OK) return st;
-  if (splitk == 0 && p.splitk > 1 && (ws == nullptr || ws_bytes < p.workspace_bytes)) {
-    st = fg_plan(M, N, K, FG_W_KN, 1, &p);
-    if (st != FG_OK) return st;
-  }
   return fg::run_gemm(A, W, C, M, N, K, accumulate, p, ws, ws_bytes, static_cast<hipStream_t>(stream),
                       0, nullptr, ldw);
 }
@@ -292,7 +291,7 @@ int fg_gemm_f16_bias_act(const void* A, const void* W, const void* bias, int act
   fg_plan_t p;
   int st;
   if (plan == nullptr) {
-    st = fg_plan(M, N, K, w_layout, splitk, &p);
+    st = fg::plan_for_workspace(M, N, K, w_layout, splitk, ws, ws_bytes, &p);
     if (st != FG_OK) return st;
     plan = &p;
   } else {

@@ -178,8 +178,8 @@ int fg_gemm_f16_planned(const void* A, const void* W, void* C, int M, int N, int
  * C = act(A·W + bias): the same kernels with the bias add and the activation applied in fp32 to
  * the finished sum (after the split-K reduction when there is one), before the single rounding
  * to fp16.  bias: fp16 [N], one value per output column, or NULL.  act: FG_ACT_*.  plan: NULL for
- * the library's choice (then `splitk` is honoured as in fg_gemm_f16), or a caller-edited plan as
- * in fg_gemm_f16_planned.  Always overwrites C.
+ * the library's choice (then `splitk` and a missing workspace are as in fg_gemm_f16), or a
+ * caller-edited plan as in fg_gemm_f16_planned.  Always overwrites C.
  *
  * No counterpart in the reference, whose operators stop at the product: the up-projection of
  * its DiT feed-forward pair (16 x 3072 x 12288, then 16 x 12288 x 3072) would be followed by a

@@ -154,3 +154,28 @@ def test_pybind_operators_and_ffn_pair(device):
     Ad, Wd = A.to(device), W1t.to(device)
     assert L.fg_gemm_f16_bias_act(ptr(Ad), ptr(Wd), None, 9, ptr(C2), M, N1, K, NK, 0, None, None, 0,
                                   stream_ptr()) == capi.FG_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("M", [8, 33, 48])
+def test_without_a_workspace_the_call_runs_unsplit(device, layout, M):
+    # the library's plan splits; without a workspace, or with too small a one, the call gives what a
+    # forced split of one gives
+    L = capi.lib()
+    N, K = 1024, 8192
+    assert layout == NK and M == 8 or capi.plan(M, N, K, layout).splitk > 1
+    g = gen(350 + M)
+    A = normal((M, K), g).to(device)
+    W = normal((K, N) if layout == KN else (N, K), g, 0.02).to(device)
+    bias = normal((N,), g).to(device)
+    small = torch.zeros(1024, dtype=torch.uint8, device=device)
+    out = []
+    for splitk, ws in ((1, None), (0, None), (0, small)):
+        C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
+        st = L.fg_gemm_f16_bias_act(ptr(A), ptr(W), ptr(bias), capi.ACT_IDS["gelu"], ptr(C), M, N, K, layout, splitk,
+                                    None, ptr(ws), 0 if ws is None else ws.numel(), stream_ptr())
+        capi.check(st, "fg_gemm_f16_bias_act")
+        out.append(C.cpu().numpy())
+    ref = oracle.gemm_bias_act(A.cpu().numpy(), W.cpu().numpy(), layout, bias.cpu().numpy(), "gelu")
+    assert_close_f16(out[0], ref, "unsplit")
+    assert (out[1] == out[0]).all() and (out[2] == out[0]).all()

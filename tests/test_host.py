@@ -327,6 +327,19 @@ def test_nk_rows_of_16_mi_elements_reach_a_kernel(M, N, K):
     assert capi.lib().fg_gemm_f16(one, one, one, M, N, K, NK, 0, 1, None, 0, None) == capi.FG_ERR_LAUNCH
 
 
+@without_device
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 4096), (33, 4096, 11008), (48, 4096, 11008), (200, 1024, 4096)])
+def test_no_entry_point_needs_a_workspace_for_the_librarys_plan(layout, M, N, K):
+    L = capi.lib()
+    one = ctypes.c_void_p(16)
+    for ws, size in ((None, 0), (one, 1024)):
+        assert L.fg_gemm_f16(one, one, one, M, N, K, layout, 0, 0, ws, size, None) == capi.FG_ERR_LAUNCH
+        assert L.fg_gemm_f16_bias_act(one, one, None, 0, one, M, N, K, layout, 0, None, ws, size, None) == capi.FG_ERR_LAUNCH
+        assert L.fg_gemm_f16_bias_act(one, one, None, 0, one, M, N, K, layout, 3, None, ws, size, None) == capi.FG_ERR_WORKSPACE
+    assert layout == NK or L.fg_gemm_f16_pitched(one, one, one, M, N, K, N + 128, 0, 0, None, 0, None) == capi.FG_ERR_LAUNCH
+
+
 # ---- pybind11 surface ---------------------------------------------------------------------------
 REFERENCE_NAMES = {
     # backend/cuda/hk/edgemm.h:4-14
