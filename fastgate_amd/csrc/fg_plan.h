@@ -14,9 +14,11 @@ bool kn_dot2_supported(int m_block, int unroll);
 bool kn_mfma_supported(int unroll);
 
 // Tiles of the kernel for more than 16 rows (fg_kernels_tile.hip): rows and columns of C per
-// workgroup, k per step.  tile_form returns the id of the form a plan runs in, or -1 for a plan that
-// takes another kernel; [N,K] plans ask for the kernel with m_block 32 and tile_n 64, [K,N] plans
-// of FG_KERNEL_KN_MFMA take it whenever M > 16.
+// workgroup, k per step.  A plan names its form in `stagger` (kTileStagger + id), which that kernel has
+// no other use for; plan_finish fills it in where it is open.  tile_form returns the id of the form a
+// finished plan runs in, or -1 for a plan that takes another kernel: it looks at the plan and at what
+// the form needs of the shape, and at nothing that can change from call to call.
+constexpr int kTileStagger = 2;
 struct TileForm {
   int rows, cols, bk;
 };

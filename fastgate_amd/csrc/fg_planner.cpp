@@ -45,6 +45,25 @@ bool tile_form_info(int form, TileForm* out) {
   return true;
 }
 
+// What a form needs of a shape, and all that the launch relies on: whole tiles, whole steps, and byte
+// offsets inside a tile's rows (k-contiguous ones) of 32 bits.
+static bool tile_fits(int form, int N, int K) {
+  TileForm t;
+  return tile_form_info(form, &t) && N % t.cols == 0 && K % t.bk == 0 &&
+         2ull * K * std::max(t.rows, t.cols) < (1ull << 32);
+}
+
+// Plans that may run as the tiled kernel: [N,K] plans that ask for it, any [K,N] MFMA plan.
+static bool tile_named(int M, const fg_plan_t& p) {
+  return M > 16 && (p.kernel == FG_KERNEL_KN_MFMA ||
+                    (p.kernel == FG_KERNEL_NK_MFMA_R && p.m_block == 32 && p.tile_n == 64));
+}
+
+int tile_form(int M, int N, int K, const fg_plan_t& p) {
+  const int form = p.stagger - kTileStagger;
+  return tile_named(M, p) && tile_fits(form, N, K) ? form : -1;
+}
+
 namespace {
 
 // Compute units the rules aim at.  The rules were fitted on 256 (MI355X); the C ABI sets the
@@ -121,8 +140,7 @@ int pick_tile(int M, int N, int K, bool kn, int splitk, int* split_out) {
   double best_us = 0.0;
   for (int f = 0; f < kTileFormCount; ++f) {
     const TileForm& t = kTileForms[f];
-    // byte offsets inside a tile are 32 bits
-    if (N % t.cols || K % t.bk || 2ull * K * std::max(t.rows, t.cols) >= (1ull << 32)) continue;
+    if (!tile_fits(f, N, K)) continue;
     const TileCost& c = kTileCosts[kn][f];
     for (int S : kSplits) {
       if (splitk > 0 && S > 1) break;
@@ -159,6 +177,15 @@ int finish_plan(int M, int N, int K, fg_plan_t* p) {
           : 4;
   if (p->splitk < 1 || p->waves < 1 || p->waves > max_waves || (p->waves & (p->waves - 1))) {
     return FG_ERR_INVALID_ARG;
+  }
+  // A plan that does not say which form it means (made by hand, or for another shape) is given the one the
+  // library takes now, and keeps it: what a plan runs as must not change with the compute units the
+  // library counts, between here and the launch or from one process to the next.
+  if (tile_named(M, *p) && tile_form(M, N, K, *p) < 0) {
+    const bool kn = p->kernel == FG_KERNEL_KN_MFMA;
+    int split;
+    const int form = !kn || tile_wins(M, N, K, FG_W_KN) ? pick_tile(M, N, K, kn, p->splitk, &split) : -1;
+    if (form >= 0) p->stagger = kTileStagger + form;
   }
   switch (p->kernel) {
     case FG_KERNEL_NK_DOT2:
@@ -398,7 +425,9 @@ int make_plan(int M, int N, int K, int w_layout, int splitk, fg_plan_t* p) {
     q.m_block = kn ? 16 : 32;
     q.band = kn ? 0 : 128;
     q.waves = 8, q.unroll = 1, q.fused = 1;
-    if (pick_tile(M, N, K, kn, splitk, &q.splitk) >= 0 && finish_plan(M, N, K, &q) == FG_OK) {
+    const int form = pick_tile(M, N, K, kn, splitk, &q.splitk);
+    q.stagger = kTileStagger + form;
+    if (form >= 0 && finish_plan(M, N, K, &q) == FG_OK) {
       *p = q;
       return FG_OK;
     }
@@ -884,14 +913,6 @@ void set_xccs(int x) {
   if (x >= 1 && x <= 64) kXccs = x;
 }
 int xccs() { return kXccs; }
-
-int tile_form(int M, int N, int K, const fg_plan_t& p) {
-  const bool kn = p.kernel == FG_KERNEL_KN_MFMA;
-  if (!kn && (p.kernel != FG_KERNEL_NK_MFMA_R || p.m_block != 32 || p.tile_n != 64)) return -1;
-  if (!tile_wins(M, N, K, kn ? FG_W_KN : FG_W_NK)) return -1;
-  int split;
-  return pick_tile(M, N, K, kn, p.splitk < 1 ? 1 : p.splitk, &split);
-}
 
 int plan_validate_shape(int M, int N, int K, int w_layout) { return validate_shape(M, N, K, w_layout); }
 int plan_make(int M, int N, int K, int w_layout, int splitk, fg_plan_t* p) {

@@ -93,15 +93,18 @@ typedef struct fg_plan_t {
   int tile_n;   /* output columns per workgroup; FG_KERNEL_NK_MFMA_R takes 16, 32, 48, 64 or,
                    with band = 128, 8 waves and no split, any divisor of N from 17 to 47  */
   int m_block;  /* rows of A per workgroup (grid.y = ceil(M / m_block)).  More than 16 rows:
-                   FG_KERNEL_NK_MFMA_R with m_block 32 and tile_n 64, and FG_KERNEL_KN_MFMA, run
-                   as the tiled kernel where the library's plans use it; that picks its own tile
-                   from (M, N, K, splitk), and grid and block here are those of the named form   */
+                   FG_KERNEL_NK_MFMA_R with m_block 32 and tile_n 64, and FG_KERNEL_KN_MFMA where
+                   the library's plans use it, run as the tiled kernel; its tile is in `stagger`,
+                   and grid and block here are those of the named kernel's own tile              */
   int waves;    /* wavefronts per workgroup; they interleave over K, reduced in LDS   */
   int unroll;   /* independent 16-byte load groups in flight per lane and step        */
   int stream_w; /* 1 = weight loads carry the non-temporal hint                       */
   int stagger;  /* K-interleaved [N,K] kernels start each workgroup at its own K step:
                    0 = (workgroup id / 8) % steps, spread within every XCD (default);
-                   1 = workgroup id % steps, one K band per XCD (only with 8 steps)  */
+                   1 = workgroup id % steps, one K band per XCD (only with 8 steps).
+                   Tiled kernel (see m_block): 2 + the number of its tile, filled by fg_plan and,
+                   where another value stands, by fg_gemm_f16_planned with the library's choice;
+                   a plan keeps its tile whatever compute units the library counts later         */
   int band;     /* FG_KERNEL_NK_MFMA_R only: bytes of K per weight row and step, 128, 256 or
                    512 (0 = 256 * unroll); a narrower band halves the activation bytes a
                    32-column tile re-reads, a wider one halves the load instructions   */

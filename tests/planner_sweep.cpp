@@ -71,6 +71,30 @@ static void check(int M, int N, int K, int layout, int splitk) {
   fg_plan_t q = p;
   REQUIRE(fg::plan_finish(M, N, K, &q) == FG_OK);
   REQUIRE(std::memcmp(&q, &p, sizeof(p)) == 0);
+  // ... and so it does when the library counts other compute units than the plan was made for, down to
+  // the form of the tiled kernel
+  const int planned_for = fg::compute_units(), form = fg::tile_form(M, N, K, p);
+  for (int cus : {304, 64}) {
+    fg::set_compute_units(cus);
+    const int finished = fg::plan_finish(M, N, K, &q), same = fg::tile_form(M, N, K, p) == form;
+    fg::set_compute_units(planned_for);
+    REQUIRE(finished == FG_OK && same);
+    REQUIRE(std::memcmp(&q, &p, sizeof(p)) == 0);
+  }
+  if (p.kernel == FG_KERNEL_NK_MFMA_R && p.m_block == 32 && p.tile_n == 64) {
+    REQUIRE(form >= 0);  // the row-load kernel has no such tile
+  }
+  if (form >= 0) {
+    fg::TileForm t;
+    REQUIRE(M > 16 && fg::tile_form_info(form, &t) && N % t.cols == 0 && K % t.bk == 0);
+    REQUIRE(2ull * K * (t.rows > t.cols ? t.rows : t.cols) < (1ull << 32));  // byte offsets inside a tile
+    if (p.splitk > 1 && p.fused == 1) REQUIRE((long long)(N / t.cols) * ((M + t.rows - 1) / t.rows) <= fg::kWsMaxTiles);
+    // a plan that leaves the form open gets one that is as good as this, and keeps it
+    q = p;
+    q.stagger = 0;
+    REQUIRE(fg::plan_finish(M, N, K, &q) == FG_OK);
+    REQUIRE(std::memcmp(&q, &p, sizeof(p)) == 0);
+  }
   switch (p.kernel) {
     case FG_KERNEL_NK_DOT2: REQUIRE(fg::nk_dot2_supported(p.m_block, p.tile_n, p.unroll)); break;
     case FG_KERNEL_NK_MFMA4: REQUIRE(fg::nk_mfma4_supported(p.m_block, p.tile_n, p.unroll)); break;
@@ -93,7 +117,7 @@ int main(int argc, char** argv) {
   for (int v : {4224, 4992, 5504, 6912, 10752, 11008, 13824, 14336 + 128, 28672 + 128, 32768 - 128}) dims.push_back(v);
   std::vector<int> ms;
   for (int m = 1; m <= 17; ++m) ms.push_back(m);
-  for (int m : {24, 31, 32, 33, 48, 64}) ms.push_back(m);
+  for (int m : {24, 31, 32, 33, 48, 64, 128, 300}) ms.push_back(m);
   const int splits_all[] = {0, 1, 2, 3, 5, 8, 16, 31, 32, 64};
   for (int cus : {256, 304, 64}) {  // the fitted part, a larger and a much smaller one
     fg::set_compute_units(cus);
@@ -117,6 +141,10 @@ int main(int argc, char** argv) {
     check(1, 128 * 16384, 128, layout, 0);
     check(1, 128, 128 * 16384, layout, 0);
     check(16, 1 << 20, 1 << 10, layout, 64);
+    // rows of 2^24 and 2^25 elements: a tile's offsets leave 32 bits, one form after the other
+    for (int M : {1, 16, 17, 32, 33, 64, 128, 300})
+      for (int K : {(1 << 23), (1 << 24) - 128, (1 << 24), (1 << 24) + 128, (1 << 25) - 128, (1 << 25), (1 << 26)})
+        for (int N : {128, 1024, 4096}) check(M, N, K, layout, 0);
   }
   std::printf("%lld plans checked\n", checked);
   return 0;

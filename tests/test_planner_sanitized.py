@@ -1,5 +1,5 @@
 """The launch planner (fastgate_amd/csrc/fg_planner.cpp, plain C++) built for the host with
-AddressSanitizer and UndefinedBehaviorSanitizer and swept over M = 1..64, every N and K that is a
+AddressSanitizer and UndefinedBehaviorSanitizer and swept over M = 1..300, every N and K that is a
 multiple of 128 up to 8192 (of 512 up to 32768, plus the odd projection sizes), both weight
 layouts, library plans and forced splits up to 64, for 256, 304 and 64 compute units: no
 undefined behaviour, and every plan launchable (tests/planner_sweep.cpp lists the conditions)."""
