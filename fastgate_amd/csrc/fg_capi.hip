@@ -76,9 +76,7 @@ int run_gemm(const void* A, const void* W, void* C, int M, int N, int K, int acc
       a.accumulate |= kFlagXcdLocal | (p.fused == 4 ? kFlagPretendForeign : 0);
     }
   }
-  // [K,N] rows so far apart that a step's offsets leave 32 bits stay with the 16-row kernel; of [N,K]
-  // weights only a tile's rows lie in one offset, which tile_form looks at itself
-  const int form = !kn || 256ull * ldw < (1ull << 32) ? tile_form(M, N, K, p) : -1;
+  const int form = tile_form(M, N, K, p);
   (void)hipGetLastError();
   bool ok = false;
   if (form >= 0) ok = launch_tile(form, kn, p, a, s);

@@ -62,7 +62,9 @@ struct TileArgs {
   int ntiles, mblocks, splitk, xccs;
 };
 
-template <bool KN, int BM, int BN, int BK, int WM, int WN, int WK, int P>
+// FAR: [K,N] rows so far apart that the offsets over the rows of a step leave 32 bits (16 Mi elements and
+// more); the same steps and sums with 64-bit addresses for the weights.
+template <bool KN, bool FAR, int BM, int BN, int BK, int WM, int WN, int WK, int P>
 __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int TM = BM / WM, TN = BN / WN;  // wave tile
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   const int s0 = (int)((long long)steps * z / S), count = (int)((long long)steps * (z + 1) / S) - s0;
 
   // Where this thread's pieces come from (bytes from the tile's first row and the step's first k)
-  // and go to.  All loads are buffer loads: activation rows beyond M lie behind the descriptor's
+  // and go to.  All loads are buffer loads (FAR's weights apart): activation rows beyond M lie behind the descriptor's
   // end and read as zeros, and a step behind the last one has an empty descriptor.  No load sits
   // behind a branch, so the number in flight is the same on every path and the waits are exact; with
   // the loads in branches the compiler waits for all of them before every park (M = 256, N = 13824,
@@ -137,17 +139,23 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   int step = count > 0 ? tile % count : 0, issued = 0;
   auto load = [&](u32x4(&a)[AI], u32x4(&w)[WI]) {
     constexpr int kNonTemporal = 2;  // the nt bit of a buffer load's cache policy
-    const int k0 = (s0 + step) * BK;
-    step = step + 1 == count ? 0 : step + 1;
     const bool live = issued++ < count;
+    const int k0 = (s0 + (FAR && !live ? 0 : step)) * BK;
+    step = step + 1 == count ? 0 : step + 1;
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t*>(Wt + (KN ? (size_t)k0 * t.ldw : (size_t)k0)), 0,
         (int)(live ? w_bytes - (KN ? 0u : (unsigned)k0 * 2u) : 0u), 0x00020000);
     const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t*>(At + k0), 0, (int)(live ? a_bytes - (unsigned)k0 * 2u : 0u), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < WI; ++i)
-      w[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)w_off[i], 0, kNonTemporal));
+    for (int i = 0; i < WI; ++i) {
+      if constexpr (FAR) {  // (a step behind the last one reads the first again; it is never multiplied)
+        const int c = i * NT + tid;
+        w[i] = load16<true>(Wt + (size_t)(k0 + c / WPR) * t.ldw + c % WPR * 8);
+      } else {
+        w[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)w_off[i], 0, kNonTemporal));
+      }
+    }
 #pragma unroll
     for (int i = 0; i < AI; ++i)
       a[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, (int)a_off[i], 0, 0));
@@ -338,11 +346,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   }
 }
 
-template <bool KN, int BM, int BN, int BK, int WM, int WN, int WK, int P>
+template <bool KN, bool FAR, int BM, int BN, int BK, int WM, int WN, int WK, int P>
 void tile_go(const TileArgs& t, hipStream_t s) {
   const int units = t.ntiles * t.splitk;
   const unsigned grid = (unsigned)((units + t.xccs - 1) / t.xccs * t.xccs) * (unsigned)t.mblocks;
-  hipLaunchKernelGGL((tile_kernel<KN, BM, BN, BK, WM, WN, WK, P>), dim3(grid),
+  hipLaunchKernelGGL((tile_kernel<KN, FAR, BM, BN, BK, WM, WN, WK, P>), dim3(grid),
                      dim3(64 * WM * WN * WK), 0, s, t);
 }
 
@@ -355,10 +363,12 @@ bool launch_tile(int form, bool kn, const fg_plan_t& p, const GemmArgs& a, hipSt
              a.ws, a.counters, a.bias, a.M, a.N, a.K, a.accumulate, a.ldw,
              a.N / f.cols, (a.M + f.rows - 1) / f.rows, p.splitk, a.xccs > 0 ? a.xccs : 1};
   if (((long long)t.ntiles * t.splitk + t.xccs) * t.mblocks > 0x7fffffffll) return false;
-#define FG_TILE(ID, BM, BN, BK, WM, WN, WK, P)                \
-  case ID:                                                          \
-    if (kn) tile_go<true, BM, BN, BK, WM, WN, WK, P>(t, s);     \
-    else tile_go<false, BM, BN, BK, WM, WN, WK, P>(t, s);       \
+  const bool far = kn && 2ull * f.bk * a.ldw >= (1ull << 32);
+#define FG_TILE(ID, BM, BN, BK, WM, WN, WK, P)                       \
+  case ID:                                                           \
+    if (far) tile_go<true, true, BM, BN, BK, WM, WN, WK, P>(t, s);   \
+    else if (kn) tile_go<true, false, BM, BN, BK, WM, WN, WK, P>(t, s); \
+    else tile_go<false, false, BM, BN, BK, WM, WN, WK, P>(t, s);     \
     return true
   switch (form) {
     FG_TILE(0, 32, 64, 128, 1, 2, 4, 2);

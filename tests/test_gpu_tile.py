@@ -175,3 +175,37 @@ def test_nk_rows_of_16_mi_elements(device, M):
         capi_gemm(A, W, C[:M], NK, splitk=splitk)
         assert torch.equal(C[:M], want.half()), splitk
         assert bool((C[M] == -7.0).all())
+
+
+@pytest.mark.parametrize("M", [33, 130])
+def test_rows_32_mib_apart_give_the_dense_result(device, M):
+    # a pitch whose offsets over the rows of a step leave 32 bits: the same tile, split and order of sums
+    N, K, ldw = 8320, 640, 1 << 24
+    A, W = _inputs(M, N, K, KN, device)
+    wide = torch.empty((K - 1) * ldw + N, dtype=torch.half, device=device)
+    torch.as_strided(wide, (K, N), (ldw, 1)).copy_(W)
+    ws = torch.zeros(1 << 26, dtype=torch.uint8, device=device)
+    for splitk in (0, 1, 2, 7):  # seven splits of five or ten steps: some have one step, some two
+        dense = torch.empty((M, N), dtype=torch.half, device=device)
+        p = capi_gemm(A, W, dense, KN, splitk=splitk)
+        assert p.workspace_bytes <= ws.numel()
+        _close(dense, _product(A, W, KN), "dense")
+        C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
+        st = capi.lib().fg_gemm_f16_pitched(ptr(A), ptr(wide), ptr(C), M, N, K, ldw, 0, splitk, ptr(ws), ws.numel(),
+                                            stream_ptr())
+        assert st == capi.FG_OK and torch.equal(C, dense), splitk
+
+
+def test_16_mi_columns(device):
+    # dense [K,N] weights as far apart: windows of columns against the product
+    M, N, K = 17, 1 << 24, 512
+    g = torch.Generator(device=device)
+    g.manual_seed(9200)
+    A = torch.randint(-2, 3, (M, K), generator=g, device=device).half()
+    W = torch.empty((K, N), dtype=torch.half, device=device)
+    for k in range(0, K, 64):
+        W[k:k + 64] = torch.randint(-3, 4, (64, N), generator=g, dtype=torch.int8, device=device)
+    C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
+    capi_gemm(A, W, C, KN)
+    for n in range(0, N, 1 << 21):
+        assert torch.equal(C[:, n:n + (1 << 21)], _product(A, W[:, n:n + (1 << 21)], KN).half()), n
