@@ -24,10 +24,10 @@ namespace {
 
 int check_launch() { return hipGetLastError() == hipSuccess ? FG_OK : FG_ERR_LAUNCH; }
 
-// The planner's rules and the [K,N] kernels' band spreading count compute units.  The entry points
-// that launch read the current device's count once, before they plan; fg_plan and
-// fg_workspace_bytes never call into the HIP runtime and plan for the count the library holds
-// at that moment (MI355X's 256 until a launch or fg_set_compute_units changed it).
+// The planner's rules, the [K,N] kernels' band spreading and the panel kernels' rules count compute
+// units.  The entry points that launch read the current device's count once, before they plan;
+// fg_plan and fg_workspace_bytes never call into the HIP runtime and plan for the count the library
+// holds at that moment (MI355X's 256 until a launch or fg_set_compute_units changed it).
 std::atomic<bool> g_cus_pinned{false};  // fg_set_compute_units was called: keep the caller's count
 void read_compute_units() {
   static std::once_flag once;
@@ -328,6 +328,7 @@ int fg_gemv_w4a16(const void* Wq4, const void* x, const void* scale, float scala
   if ((reinterpret_cast<uintptr_t>(Wq4) | reinterpret_cast<uintptr_t>(x)) & 15) {
     return FG_ERR_INVALID_ARG;
   }
+  fg::read_compute_units();
   fg::W8A16Args a{Wq4, x, scale, scalar_scale, zero_point, y, M, N, K};
   (void)hipGetLastError();
   if (!fg::launch_w4a16(a, static_cast<hipStream_t>(stream))) return FG_ERR_UNSUPPORTED;
@@ -342,6 +343,7 @@ int fg_gemv_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N,
   if ((reinterpret_cast<uintptr_t>(Wq) | reinterpret_cast<uintptr_t>(xq)) & 15) {
     return FG_ERR_INVALID_ARG;
   }
+  fg::read_compute_units();
   (void)hipGetLastError();
   if (!fg::launch_i8i8_i32(Wq, xq, acc, M, N, K, static_cast<hipStream_t>(stream))) {
     return FG_ERR_UNSUPPORTED;

@@ -897,7 +897,8 @@ static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
   // (M=4 N=14336 K=4096 10.7 / 9.3; N=12288 K=3072, 384 workgroups, 7.6 / 8.6 the other way).  KC: the
   // smallest that holds K; sixteen waves share the largest panels (K=14336 11.9 / 11.5 with eight).
   const int t32 = a.N / 32;
-  const bool wide = t32 >= 224 && 8 * t32 >= 7 * ((t32 + 255) / 256 * 256);
+  const int cus = compute_units();
+  const bool wide = 8 * t32 >= 7 * ((t32 + cus - 1) / cus * cus);
   if (a.K <= 2048) { if (wide) FG_W4_X(2048, 2, 8); else FG_W4_X(2048, 1, 8); }
   else if (a.K <= 4096) { if (wide) FG_W4_X(4096, 2, 8); else FG_W4_X(4096, 1, 8); }
   else if (a.K <= 6144) { if (wide) FG_W4_X(6144, 2, 8); else FG_W4_X(6144, 1, 8); }
@@ -937,16 +938,23 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
                     hipStream_t s) {
   auto* W = static_cast<const int8_t*>(Wq);
   auto* X = static_cast<const int8_t*>(xq);
-  // Two to four rows: four weight rows a workgroup, one 1 KB piece of each in flight a wave, and three or
-  // four waves, whichever leaves fewer of the last step's waves without a piece -- except whole
-  // multiples of 8 KB rows, which two pieces of eight rows on four waves divide evenly (M=4, us, eight rows
-  // and two pieces / this: N = K = 5120 8.3 / 7.5, N=14336 K=4096 14.3 / 12.3, N=12288 K=3072 11.0 / 9.0,
-  // N=3072 K=9088 8.5 / 7.7, N=4096 K=11008 12.1 / 10.9, but N = K = 8192 13.6 / 13.9).  Narrow outputs keep two
-  // pieces in flight, their workgroups do not fill the chip (N=2048 K=14336 M=4 7.9 / 8.5), and the
-  // longest rows are level (N=4096 K=14336 M=4 12.8 / 13.0).
+  // Two to four rows.  One form has four weight rows a workgroup, one 1 KB piece of each in flight a
+  // wave, and three or four waves, whichever leaves fewer of the last step's waves without a piece; the
+  // other, below, eight rows (four for narrow outputs), two pieces a wave, four waves.  One after the other in
+  // a replayed graph, us, the second form / the first:
+  //  * two rows: the first throughout (N = K = 5120 7.2 / 6.5, N = K = 8192 12.6 / 12.1, N=28672 K=8192 36.5 /
+  //    34.7, K=12288 52.0 / 51.7), three rows too (8.2 / 7.3, 13.5 / 13.2, 37.0 / 37.1, 53.4 / 54.9);
+  //  * four rows: the first (N = K = 5120 8.4 / 7.5, N=14336 K=4096 14.6 / 12.8, N=12288 K=8704 21.8 / 20.9,
+  //    N=16384 K=11008 33.6 / 32.6) but for eight and twelve pieces against wide outputs, where the second's
+  //    waves all have as many (N=8192 K=7936 13.7 / 14.1, N=28672 K=7936 36.0 / 39.5, N = K = 8192 13.9 / 14.1;
+  //    N = K = 12288 26.0 / 28.2, N=28672 K=11520 52.0 / 55.9; N=5120 K=8192 11.1 / 10.2, N=11008 K=12288
+  //    25.0 / 25.2);
+  //  * narrow outputs keep the second, their workgroups do not fill the chip (N=2048 K=6144 M=4 5.3 /
+  //    5.4, K=14336 7.9 / 8.5), and so do the longest rows (N=4096 K=14336 M=4 12.8 / 13.0).
   if (MB == 2 || MB == 4) {
     const int pieces = (K / 16 + 63) / 64;
-    if (N > 2048 && K <= 12288 && K % 8192 != 0) {
+    const bool full_steps = M == 4 && pieces >= 8 && pieces % 4 == 0 && N >= 1024 * pieces;
+    if (N > 2048 && pieces <= 12 && !full_steps) {
       const int waves = pieces <= 4 ? pieces : ((pieces + 2) / 3 * 3 < (pieces + 3) / 4 * 4 ? 3 : 4);
       hipLaunchKernelGGL((i8i8_kernel<MB, 4, 1>), dim3(N / 4), dim3(64 * waves), 0, s, W, X, acc, M, N, K);
       return;
@@ -969,18 +977,23 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
 //    K=5120 24.5 / 20.7; N = K = 8192 19.1 / 16.0, N = K = 4096 8.8 / 5.9; N=4096 K=14336 16.7 / 14.9.  Not
 //    narrow outputs with long rows (N=2048 K=8192 7.7 / 8.2, K=4096 5.9 / 5.1; N=1024 K=4096 4.7 / 5.0), and
 //    not tiles that leave a third of the CUs' second round idle (N = K = 5120, 320 tiles, M=5 10.5 / 10.6).
-//  * two to four rows: short rows (M=4 N=7168 K=2048 6.1 / 5.1, N=11008 K=1024 6.2 / 4.6, N = K = 2048
-//    3.9 / 3.5), and three and four where the tiles fill the CUs exactly (N = K = 4096 6.8 / 5.7, N=4096
-//    K=6144 7.7 / 6.9, N=16384 K=4096 16.4 / 15.6; N=14336 K=4096 14.6 / 15.2).  Elsewhere 1 KB of a row a
-//    load beats 16 rows x 64 bytes (N = K = 8192 13.6 / 14.4, N = K = 5120 8.2 / 10.3).
+//  * two to four rows: short rows, the shorter the wider the output (K=1024 M=4 N=11008 5.1 / 4.7, N=28672
+//    8.1 / 8.0; K=2048 N=2048 4.0 / 3.3, N=8192 5.5 / 5.2, N=16384 8.5 / 8.4, N=28672 12.0 / 12.9; M=2 K=1024
+//    N=11008 4.4 / 4.3, N=14336 4.9 / 5.3, K=2048 N=8192 5.1 / 4.9, N=11008 6.0 / 6.4);
+//  * three and four rows with one workgroup on every CU or nearly (M=4 K=4096 N=3072 5.3 / 4.9, N=4096 6.0 /
+//    5.2; M=3 5.2 / 4.9, 5.8 / 5.2), on every CU up to K = 6144 (N=4096 M=4 7.2 / 6.9, M=3 6.8 / 6.8; N=3072 6.0 /
+//    6.6).  A second one a CU, or a longer row, and 1 KB of a row a load beats 16 rows x 64 bytes (K=4096 M=4
+//    N=8192 8.8 / 8.8, N=12288 11.5 / 12.1, N=16384 14.1 / 15.2, N=4224 6.2 / 7.5; N = K = 5120 7.5 / 10.4).
 static bool i8_panel(int M, int N, int K) {
   if (M < 2 || N < 2048 || K > 16384) return false;
-  const int tiles = N / 16;
+  const int tiles = N / 16, cus = compute_units();
   if (M >= 5) {
-    const bool even = 10 * tiles >= 7 * ((tiles + 255) / 256 * 256);
+    const bool even = 10 * tiles >= 7 * ((tiles + cus - 1) / cus * cus);
     return K <= 4096 || (N > 2048 && even);
   }
-  return K <= 2048 || (M >= 3 && K <= 6144 && (tiles == 256 || tiles == 512 || tiles == 1024) && (K <= 4096 || tiles == 256));
+  if (M == 2) return K <= 512 || (K <= 2048 && N <= 8192);
+  if (K <= 1536 || (K <= 2048 && N <= 16384)) return true;
+  return tiles <= cus && 4 * tiles >= 3 * cus && K <= (tiles == cus ? 6144 : 4096);
 }
 
 bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N, int K,
@@ -991,15 +1004,17 @@ bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N,
     auto* X = static_cast<const int8_t*>(xq);
 #define FG_I8_X(XR, KC, NW) \
   hipLaunchKernelGGL((i8i8_x_kernel<XR, KC, NW>), dim3(N / 16), dim3(64 * NW), 0, s, W, X, acc, M, N, K)
-#define FG_I8_X_KC(XR)                            \
-  if (K <= 2048) FG_I8_X(XR, 2048, 8);             \
-  else if (K <= 4096) FG_I8_X(XR, 4096, 8);        \
-  else if (K <= 6144) FG_I8_X(XR, 6144, 8);        \
-  else if (K <= 8192) FG_I8_X(XR, 8192, 8);        \
-  else if (K <= 12288) FG_I8_X(XR, 12288, 16);     \
-  else FG_I8_X(XR, 16384, 16)
-    if (M <= 4) { FG_I8_X_KC(4); } else { FG_I8_X_KC(8); }
-#undef FG_I8_X_KC
+    if (M <= 4) {  // up to K = 6144, see i8_panel
+      if (K <= 2048) FG_I8_X(4, 2048, 8);
+      else if (K <= 4096) FG_I8_X(4, 4096, 8);
+      else if (K <= 6144) FG_I8_X(4, 6144, 8);
+      else return false;
+    } else if (K <= 2048) FG_I8_X(8, 2048, 8);
+    else if (K <= 4096) FG_I8_X(8, 4096, 8);
+    else if (K <= 6144) FG_I8_X(8, 6144, 8);
+    else if (K <= 8192) FG_I8_X(8, 8192, 8);
+    else if (K <= 12288) FG_I8_X(8, 12288, 16);
+    else FG_I8_X(8, 16384, 16);
 #undef FG_I8_X
   } else if (M == 1) {
     i8i8_go<1>(Wq, xq, acc, M, N, K, s);

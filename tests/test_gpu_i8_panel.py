@@ -1,6 +1,8 @@
-"""int8 x int8 products through the kernel that holds two to eight activation rows in LDS as one panel: K at
-and beside the panel sizes, both panel heights, whole int8 range, exact to the bit; nothing is written
-behind the result."""
+"""int8 x int8 products of two to eight activation rows, which the kernel that holds them in LDS as one panel
+and the v_dot4 kernel share between them: K at and beside the panel sizes (five rows and more run the
+panel there, two to four up to K = 2048, three and four against 4096 outputs up to 6144, the v_dot4
+kernel the rest), sizes on both sides of each line of the rule, whole int8 range, exact to the bit;
+nothing is written behind the result."""
 import pytest
 import torch
 
@@ -38,4 +40,23 @@ def test_few_rows_beside_the_panel_are_exact(device, N, K):
         acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
         assert capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr()) == capi.FG_OK
         assert torch.equal(acc[:M], (x.double() @ W.double().t()).round().int()), (M, N, K)
+        assert bool((acc[M] == -3).all())
+
+
+# both sides of every line between the panel, one piece a wave, and two pieces a wave
+@pytest.mark.parametrize("N,K", [(8192, 2048), (8320, 2048), (14336, 512), (14336, 640), (28672, 1536), (28672, 1664),
+                                 (16384, 2048), (16512, 2048), (3072, 4096), (2944, 4096), (3072, 4224), (4096, 6144),
+                                 (4096, 6272), (4224, 4096), (8192, 4096), (16384, 4096), (8192, 7296), (8064, 8192),
+                                 (8192, 8192), (12288, 11264), (12288, 11392), (12160, 11392), (12288, 12288),
+                                 (2176, 12288), (2176, 12416)])
+def test_lines_of_the_rule_are_exact(device, N, K):
+    g = torch.Generator(device=device)
+    g.manual_seed(9800 + N + K)
+    W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)
+    W64 = W.double().t()
+    for M in (2, 3, 4):
+        x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=device)
+        acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
+        assert capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr()) == capi.FG_OK
+        assert torch.equal(acc[:M], (x.double() @ W64).round().int()), (M, N, K)
         assert bool((acc[M] == -3).all())
