@@ -68,3 +68,28 @@ def test_broken_rows_stay_alone(device, N, K):
     w = (Wd[:, 2] >> 4).cpu().numpy().astype(np.float32) - 8.0  # k = 5: the high nibble of byte 2
     assert (np.isnan(got[1]) == (w == 0)).all() and (np.sign(got[1][w != 0]) == np.sign(w[w != 0])).all()
     assert np.isinf(got[1][w != 0]).all() and np.isnan(got[3]).all()
+
+
+@pytest.mark.parametrize("unit", [2.0 ** -24, 32.0])  # subnormal activations up to 511 units; the largest halves
+@pytest.mark.parametrize("N,K", [(2176, 512), (2176, 4096), (7168, 2048), (2176, 12288)])
+def test_smallest_and_largest_activations_are_exact(device, N, K, unit):
+    # 512 activations a row are not zero.  In units, |x| <= 2047 and weights below 16 keep the sum of all
+    # magnitudes below 512 * 2047 * 15 < 2^24, so every partial sum is exact in fp32 in any order and the
+    # only rounding is the last one
+    g = gen(9900 + K + int(unit))
+    Wd = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8)
+    W = torch.stack((Wd & 15, Wd >> 4), dim=-1).flatten(1).numpy().astype(np.int64) - 8
+    scalar = 1.0 if unit < 1 else 2.0 ** -14
+    for M in (2, 3, 4):
+        m = torch.zeros((M, K), dtype=torch.int64)
+        top = 511 if unit < 1 else 2047
+        for row in range(M):
+            at = torch.randperm(K, generator=g)[:512]
+            m[row, at] = torch.randint(1, top + 1, (512,), generator=g) * (torch.randint(0, 2, (512,), generator=g) * 2 - 1)
+            m[row, at[:64]] = top
+        x = (m.double() * unit).half()
+        assert (x.double() / unit == m.double()).all()
+        got = _run(Wd.to(device), x, None, scalar, 8.0, device)
+        want = ((m.numpy() @ W.T) * (unit * scalar)).astype(np.float32).astype(np.float16)
+        assert (want != 0).mean() > 0.99
+        assert (got == want).all(), (M, N, K)

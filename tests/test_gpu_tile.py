@@ -10,7 +10,7 @@ import torch
 
 import oracle
 from fastgate_amd import capi
-from helpers import ATOL, RTOL, assert_close_f16, capi_gemm, ptr, stream_ptr
+from helpers import ATOL, RTOL, assert_close_f16, capi_gemm, make_plan, ptr, stream_ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -209,3 +209,49 @@ def test_16_mi_columns(device):
     capi_gemm(A, W, C, KN)
     for n in range(0, N, 1 << 21):
         assert torch.equal(C[:, n:n + (1 << 21)], _product(A, W[:, n:n + (1 << 21)], KN).half()), n
+
+
+def _form(p):
+    return p.stagger - 2  # include/fastgate.h: 2 + the number of the tile
+
+
+FORMS = range(7)
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("form", FORMS)
+def test_every_form_at_the_edges_of_its_rows(device, layout, form):
+    # whole numbers, so every form and split gives the exact sum; 40 splits of 33 steps or fewer leave
+    # workgroups without a step
+    N, K = 1280, 2176
+    for M in (17, 31, 32, 33, 63, 65, 95, 97, 127, 129, 300):
+        A, W = _inputs(M, N, K, layout, device, whole=True)
+        exact = _product(A, W, layout).half()
+        for splitk in (1, 3, 40):
+            p = make_plan(capi.FG_KERNEL_KN_MFMA, tile_n=128, m_block=16, waves=8, splitk=splitk, stagger=2 + form) if \
+                layout == KN else make_plan(capi.FG_KERNEL_NK_MFMA_R, tile_n=64, m_block=32, waves=8, splitk=splitk,
+                                            stagger=2 + form, band=128)
+            C = torch.full((M + 1, N), -7.0, dtype=torch.half, device=device)
+            capi_gemm(A, W, C[:M], layout, plan=p)
+            assert _form(p) == form  # kept: the tile fits the shape
+            assert torch.equal(C[:M], exact), (M, splitk)
+            assert bool((C[M] == -7.0).all())
+
+
+# the library's own plans, one at least for every form of either layout
+LIBRARY = [(KN, 31, 11008, 1024, 0), (KN, 24, 14336, 3072, 1), (KN, 64, 6144, 4096, 2), (KN, 96, 10240, 1024, 3),
+           (KN, 128, 11008, 3072, 4), (KN, 200, 10240, 4096, 5), (KN, 48, 28672, 1024, 6), (NK, 32, 3072, 11008, 0),
+           (NK, 17, 13824, 5120, 1), (NK, 32, 8192, 11008, 1), (NK, 31, 10240, 3072, 1), (NK, 17, 6144, 5120, 1), (NK, 64, 6144, 8192, 2),
+           (NK, 96, 10240, 3072, 3), (NK, 128, 11008, 5120, 4), (NK, 200, 13824, 5120, 5), (NK, 48, 28672, 3072, 6)]
+
+
+@pytest.mark.parametrize("layout,M,N,K,form", LIBRARY)
+def test_library_plans_of_the_tiled_kernel(device, layout, M, N, K, form):
+    for splitk in (0, 1, 2, 5):
+        p = capi.plan(M, N, K, layout, splitk)
+        if splitk == 0:
+            assert _form(p) == form, p.as_dict()
+        A, W = _inputs(M, N, K, layout, device, whole=True)
+        C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
+        capi_gemm(A, W, C, layout, plan=p)
+        assert torch.equal(C, _product(A, W, layout).half()), splitk
