@@ -18,8 +18,9 @@
  *   C      fp16 [M,N] row-major, caller allocated
  *   K, N   multiples of 128 (the reference's only documented constraint, README.md:6-12)
  *   M      any positive value: kernels of their own for M = 1..16, a tiled one beyond (one pass
- *          over the weights for up to 128 rows; weights of less than 4 Mi elements keep the small-M
- *          kernels, which read them once per 32 or 16 rows)
+ *          over the weights for up to 128 rows).  Where that did not measure ahead -- K < 512, weights
+ *          of 4 Mi elements or less in part, 17..32 rows of many [N,K] shapes -- the small-M kernels
+ *          stay, which read the weights once per 32 ([N,K]) or 16 ([K,N]) rows
  *   arithmetic: fp16 products, fp32 accumulation, one rounding to fp16 at the end
  */
 #ifndef FASTGATE_H_
@@ -251,7 +252,8 @@ int fg_gemv_w4a16(const void* Wq4, const void* x, const void* scale, float scala
                   float zero_point, void* y, int M, int N, int K, void* stream);
 
 /*
- * Integer dot stage: acc[m,n] = Σ_k int32(xq[m,k])·int32(Wq[n,k]) with v_dot4_i32_i8.
+ * Integer dot stage: acc[m,n] = Σ_k int32(xq[m,k])·int32(Wq[n,k]), with v_dot4_i32_i8 or, for five rows
+ * and more and for short rows, v_mfma_i32_16x16x64_i8 (the same sums, exact).
  * Wq int8 [N,K], xq int8 [M,K], acc int32 [M,N].  Exact for K <= 2^17.  1 <= M <= 8.
  * No counterpart in the reference (its int8 GEMV multiplies fp16 activations); this is the
  * stage whose result is compared bit for bit.
