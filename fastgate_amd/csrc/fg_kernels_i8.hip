@@ -11,6 +11,8 @@
 #include "fg_device.h"
 #include "fg_internal.h"
 
+#include <algorithm>
+
 namespace fg {
 
 // Per-channel scale of the output a thread writes at the end, fetched ahead of the weight stream
@@ -626,129 +628,178 @@ __global__ __launch_bounds__(512) void w4a16_r_kernel(const uint8_t* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------
-// w4a16, two to four activation rows: all activations of the workgroup in LDS, the weights from memory
-// straight into the MFMA operand.  A 4-row activation panel is 8 bytes a k, so all of it fits
-// LDS up to KC = 16384 k; every wave has its whole share of the tile's weight rows in flight (loads of
-// 16 rows x 64 bytes) while the panel is staged, and nothing but the decode stands between a weight's
-// arrival and its product: no LDS round trip for the weights and one memory latency a call.  Launched
-// with K <= KC.  What bounds it: launch and the two streams, weights from memory and as many or
-// twice as many panel bytes from L2 (M=4 N=4096 K=14336, 29 MB: 11.5 us, 2.6 TB/s, a plain read 5.7;
-// N=14336 K=4096 9.3); the row-load kernel above takes 13.0 and 13.2, with five operations more a word
-// and both operands through LDS.
-//  * Lane (j, g) loads 16 bytes = 32 k of row j: four words of eight nibbles.  The even nibbles of
+// w4a16, two to four activation rows: all activations in LDS as one panel (4 rows x KC k, 8 bytes a k), staged
+// once a workgroup, which then walks over column tiles of 16; the weights of a tile go from memory through
+// registers and two KB of wave-private LDS into MFMA operands.  Launched with K <= KC.
+//  * All loads are row-contiguous: eight lanes read the 128 bytes of a line.  A CU takes 64 bytes a clock
+//    that way; where neighbouring lanes sit on different rows, as the operand order of the MFMA would have it,
+//    it takes 18 (measured: reads of L2-resident data on every CU, 129 GB/s a CU against 38).
+//  * Every wave has its whole share of a tile in flight; the registers of a load are filled again, with the next
+//    tile's, as soon as it has been parked.
+//  * Lane (j, g) takes 16 bytes = 32 k of row j: four words of eight nibbles.  The even nibbles of
 //    two words make one MFMA operand (nibbles 0,4,2,6 of each), the odd ones a second: masked in
 //    place they are fp16 subnormals, n 2^-24 and n 2^-20, exactly, so five integer operations
 //    decode eight weights and two accumulators keep the two powers of two apart.
-//  * The panel lies in LDS in that order: 16-byte pieces [load][word pair][even, odd][g][row], so one
-//    operand read of a wave covers 256 contiguous bytes (the lanes of rows 4..15 repeat rows 0..3).
+//  * The panel lies in LDS in that order: 16-byte pieces [128 k][word pair][even, odd][g][row], so one
+//    operand read of a wave covers 256 contiguous bytes (the lanes of rows 4..15 repeat rows 0..3).  The rows
+//    of a group are permuted by its number: the threads that stage it have consecutive k of one row.
 //  * The row sums for the zero point are taken while the panel is staged.
+// Loads return in order, so their order counts: activations, then the scales (cold), then the weights (the scales
+// last: 0.35 us more on every call).
+// What bounds it: N=4096 K=14336 M=4 9.9 us of which a call without any load or product takes 4.3, the weights
+// 3.4 more (29 MB), activations 1.2 (115 KB a CU from L2), decode and products after the last load 1.0.  Measured
+// against the same panel with the loads in operand order and one tile a workgroup (us): N=4096 K=14336 M=4
+// 11.8 / 9.9, N = K = 8192 10.9 / 8.8, N=14336 K=4096 9.1 / 7.9, N=28672 K=2304 11.2 / 8.9, N=4096 K=4096 4.4 / 4.1.
 // ---------------------------------------------------------------------------------------
-template <int KC, int CB, int NW>
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row16_allreduce(v);
+  float s = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) s += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16 * r));
+  return s;
+}
+template <int KC, int NW>
 __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restrict__ Wq, const half_t* __restrict__ X,
                                                       const half_t* __restrict__ scale, float scalar_scale,
                                                       float zero_point, half_t* __restrict__ Y, int M, int N, int K) {
-  constexpr int LOADS = KC / 128 / NW;     // weight loads a wave
-  constexpr int GROUPS = KC / 16 / (16 * NW);    // 16-k groups of its activation row a thread
-  __shared__ u32x4 panel[KC / 2];          // 4 rows x KC halves
-  __shared__ float red[NW][CB][2][64];
-  __shared__ float xred[NW][4];
+  constexpr int PAIRS = KC / 256 / NW;           // 16 rows x 128 bytes of weights: two loads a wave
+  constexpr int SEGS = KC / 512 / (NW / 4);      // 1 KB of an activation row: one load a wave
+  static_assert(KC % (256 * NW) == 0 && KC % (128 * NW) == 0, "whole pairs and segments");
+  constexpr int STRIP = 2048;
+  constexpr bool kOwnRed = KC * 8 + NW * (STRIP + 2 * 516) <= 160 * 1024 - 64;
+  constexpr int RED = 129;                       // floats a wave hands over: two powers of two of 4 x 16 sums, one row sum
+  __shared__ u32x4 panel[KC / 2];
+  __shared__ __attribute__((aligned(16))) unsigned char strips[NW * STRIP];
+  __shared__ float own_red[kOwnRed ? 2 * NW * RED : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int j = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (16 * CB);
+  const int j = lane & 15, g = lane >> 4;        // operand order
+  const int lr = lane >> 3, lp = lane & 7;       // load order: row, 16-byte piece of its 128
   const size_t rowb = (size_t)K >> 1;
-  // scale of the output this thread writes at the end, fetched ahead of the weight stream
-  const uint32_t scale_raw = scale_fetch(scale, n0 + (tid >> 6) * 16 + (tid & 15), tid < 64 * CB);
   constexpr int kNonTemporal = 2;
-  const __amdgpu_buffer_rsrc_t wrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(Wq + (size_t)n0 * rowb), 0, (int)(16 * CB * rowb), 0x00020000);
-  const __amdgpu_buffer_rsrc_t xrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(X), 0, M * K * 2, 0x00020000);
-  constexpr int kBeyond = 0x7ffffff0;      // past both descriptors: the load returns zeros
-  const int xm = tid & 3, xq = tid >> 2;   // this thread's activation row and first group
-  const half2_t ones = {static_cast<half_t>(1.f), static_cast<half_t>(1.f)};
-  float4_t even[CB], odd[CB];
-#pragma unroll
-  for (int b = 0; b < CB; ++b) even[b] = odd[b] = float4_t{0.f, 0.f, 0.f, 0.f};
-  float xsum = 0.f;
-  auto load_of = [&](int t) { return wave + NW * t; };
-  const int loads = K >> 7;
-  u32x4 x0[GROUPS], x1[GROUPS], w[CB][LOADS];
+  constexpr int kBeyond = 0x7ffffff0;            // past the descriptors: the load returns zeros
+
   // activations first: loads return in order, and the panel must not wait for the weights
+  const int per_row = M == 2 ? NW / 2 : (M == 3 ? NW / 3 : NW / 4);  // waves that stage a row
+  const int xm = wave / per_row, xs0 = wave - xm * per_row;
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(X + (size_t)xm * K), 0, xm < M ? K * 2 : 0, 0x00020000);
+  u32x4 x[SEGS];
 #pragma unroll
-  for (int i = 0; i < GROUPS; ++i) {
-    const int q = xq + 16 * NW * i;
-    const int off = (q * 16 < K && xm < M) ? (xm * K + q * 16) * 2 : kBeyond;
-    x0[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
-    x1[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 16, 0));
+  for (int i = 0; i < SEGS; ++i)
+    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (xs0 + per_row * i) * 1024 + lane * 16, 0, 0));
+  __builtin_amdgcn_sched_barrier(0);
+
+  u32x4 w[PAIRS][2];
+  int w_off[PAIRS];
+#pragma unroll
+  for (int t = 0; t < PAIRS; ++t) {
+    const int kb = (wave + NW * t) * 128 + lp * 16;
+    w_off[t] = kb < (int)rowb ? lr * (int)rowb + kb : kBeyond;
+  }
+  const int tiles = N >> 4;
+  auto load_pair = [&](int tile, int t) {
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(Wq + (size_t)tile * 16 * rowb), 0, tile < tiles ? (int)(16 * rowb) : 0, 0x00020000);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[t][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              wrs, w_off[t] == kBeyond ? kBeyond : w_off[t] + 8 * h * (int)rowb, 0, kNonTemporal));
+  };
+  int tile = blockIdx.x;
+  // scale of the output this thread writes, ahead of the tile's weights
+  uint32_t scale_raw = scale_fetch(scale, tile * 16 + ((tid >> 2) & 15), tid < 256);
+#pragma unroll
+  for (int t = 0; t < PAIRS; ++t) {
+    load_pair(tile, t);
+    __builtin_amdgcn_sched_barrier(0);           // in this order: they are waited for one after the other
   }
   __builtin_amdgcn_sched_barrier(0);
+
+  const half2_t ones = {static_cast<half_t>(1.f), static_cast<half_t>(1.f)};
+  float xsum = 0.f;
 #pragma unroll
-  for (int t = 0; t < LOADS; ++t) {
-    const int l = load_of(t);
+  for (int i = 0; i < SEGS; ++i) {
+    const int seg = xs0 + per_row * i;
+    if (xm < M && seg * 512 < KC) {
+      const u32x4 a = x[i];
 #pragma unroll
-    for (int b = 0; b < CB; ++b) {
-      const int off = l < loads ? (16 * b + j) * (int)rowb + l * 64 + g * 16 : kBeyond;
-      w[b][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, 0, kNonTemporal));
+      for (int c = 0; c < 4; ++c) xsum = __builtin_amdgcn_fdot2(as_half2(a[c]), ones, xsum, false);
+      constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;
+      const int q = seg * 32 + (lane >> 1);      // 16-k group
+      u32x2* at = reinterpret_cast<u32x2*>(panel + (q >> 3) * 64 + (q & 1) * 32 + ((q >> 1) & 3) * 4 + (xm ^ ((q >> 3) & 3))) + (lane & 1);
+      at[0] = u32x2{__builtin_amdgcn_perm(a.z, a.x, kLow), __builtin_amdgcn_perm(a.w, a.y, kLow)};
+      at[32] = u32x2{__builtin_amdgcn_perm(a.z, a.x, kHigh), __builtin_amdgcn_perm(a.w, a.y, kHigh)};
     }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < GROUPS; ++i) {
-    const int q = xq + 16 * NW * i;
-    const u32x4 a = x0[i], b = x1[i];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      xsum = __builtin_amdgcn_fdot2(as_half2(a[c]), ones, xsum, false);
-      xsum = __builtin_amdgcn_fdot2(as_half2(b[c]), ones, xsum, false);
-    }
-    constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;
-    u32x4* at = panel + (q >> 3) * 64 + (q & 1) * 32 + ((q >> 1) & 3) * 4 + xm;
-    at[0] = u32x4{__builtin_amdgcn_perm(a.z, a.x, kLow), __builtin_amdgcn_perm(a.w, a.y, kLow),
-                  __builtin_amdgcn_perm(b.z, b.x, kLow), __builtin_amdgcn_perm(b.w, b.y, kLow)};
-    at[16] = u32x4{__builtin_amdgcn_perm(a.z, a.x, kHigh), __builtin_amdgcn_perm(a.w, a.y, kHigh),
-                   __builtin_amdgcn_perm(b.z, b.x, kHigh), __builtin_amdgcn_perm(b.w, b.y, kHigh)};
   }
   __syncthreads();
+  xsum = wave_sum(xsum);
+
+  unsigned char* const strip = strips + wave * STRIP;
+  for (int parity = 0; tile < tiles; tile += gridDim.x, parity ^= 1) {
+    float4_t even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+    const int next = tile + (int)gridDim.x;
+    const uint32_t scale_now = scale_raw;
+    scale_raw = scale_fetch(scale, next * 16 + ((tid >> 2) & 15), tid < 256 && next < tiles);
 #pragma unroll
-  for (int t = 0; t < LOADS; ++t) {        // (past the end of K: zero weights on a zero panel)
+    for (int t = 0; t < PAIRS; ++t) {
+      const int pair = wave + NW * t;
+      // the panel's operands do not wait for the weights
+      u32x4 xe[2][2], xo[2][2];
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const u32x4* at = panel + (load_of(t) * 2 + p) * 32 + g * 4 + (j & 3);
-      const u32x4 xe = at[0], xo = at[16];
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int b = 0; b < CB; ++b) {
-        const uint32_t u = w[b][t][2 * p], v = w[b][t][2 * p + 1], u8 = u >> 8, v8 = v >> 8;
-        const u32x4 we = {u & 0x000F000Fu, u8 & 0x000F000Fu, v & 0x000F000Fu, v8 & 0x000F000Fu};  // 0,4 2,6 of both
-        const u32x4 wo = {u & 0x00F000F0u, u8 & 0x00F000F0u, v & 0x00F000F0u, v8 & 0x00F000F0u};  // 1,5 3,7
-        even[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xe), as_half8(we), even[b], 0, 0, 0);
-        odd[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xo), as_half8(wo), odd[b], 0, 0, 0);
+        for (int p = 0; p < 2; ++p) {
+          const u32x4* at = panel + ((pair * 2 + u) * 2 + p) * 32 + g * 4 + ((j ^ (pair * 2 + u)) & 3);
+          xe[u][p] = at[0];
+          xo[u][p] = at[16];
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4*>(strip + h * 1024 + lr * 128 + 16 * (lp ^ lr)) = w[t][h];
+      wave_lds_sync();
+      load_pair(next, t);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {              // (past the end of K: zero weights on a zero panel)
+        const u32x4 wv = *reinterpret_cast<const u32x4*>(strip + j * 128 + 16 * ((4 * u + g) ^ (j & 7)));
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const uint32_t a = wv[2 * p], b = wv[2 * p + 1], a8 = a >> 8, b8 = b >> 8;
+          const u32x4 we = {a & 0x000F000Fu, a8 & 0x000F000Fu, b & 0x000F000Fu, b8 & 0x000F000Fu};  // 0,4 2,6 of both
+          const u32x4 wo = {a & 0x00F000F0u, a8 & 0x00F000F0u, b & 0x00F000F0u, b8 & 0x00F000F0u};  // 1,5 3,7
+          even = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xe[u][p]), as_half8(we), even, 0, 0, 0);
+          odd = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xo[u][p]), as_half8(wo), odd, 0, 0, 0);
+        }
       }
+      wave_lds_sync();
     }
-  }
-  // lanes 0..15 hold rows 0..3 of column j in registers 0..3; lanes of one activation row sit 4 apart
-#pragma unroll
-  for (int d = 4; d < 64; d <<= 1) xsum += __shfl_xor(xsum, d);
-  if (lane < 4) xred[wave][lane] = xsum;
-  if (lane < 16) {
-#pragma unroll
-    for (int b = 0; b < CB; ++b)
+    // lanes 0..15 hold rows 0..3 of column j in registers 0..3
+    float* const red = kOwnRed ? own_red + parity * NW * RED : reinterpret_cast<float*>(strips);
+    constexpr int kRedStep = kOwnRed ? RED : STRIP / 4;
+    if (lane < 16) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        red[wave][b][0][r * 16 + j] = even[b][r];
-        red[wave][b][1][r * 16 + j] = odd[b][r];
+        red[wave * kRedStep + r * 16 + j] = even[r];
+        red[wave * kRedStep + 64 + r * 16 + j] = odd[r];
       }
-  }
-  __syncthreads();
-  if (tid < 64 * CB) {
-    const int b = tid >> 6, e = tid & 63, m = e >> 4, n = n0 + 16 * b + (e & 15);
-    if (m < M) {
-      const float se = lds_sum<NW>(&red[0][b][0][e], 128 * CB, NW), so = lds_sum<NW>(&red[0][b][1][e], 128 * CB, NW);
-      const float xs = lds_sum<NW>(&xred[0][m], 4, NW);
-      float v = (se * 16777216.f + so * 1048576.f) - zero_point * xs;
-      if (not_finite(xs)) v = elementwise_dot<4>(Wq + (size_t)n * rowb, X + (size_t)m * K, K, zero_point);
-      Y[(size_t)m * N + n] = static_cast<half_t>(v * (scalar_scale * scale_value(scale_raw)));
     }
+    if (lane == 0) red[wave * kRedStep + 128] = xsum;
+    __syncthreads();
+    // four threads an output: a quarter of the waves each
+    if (tid < 256) {
+      const int e = tid >> 2, m = e >> 4, n = tile * 16 + (e & 15), part = tid & 3;
+      const float* const r = red + part * (NW / 4) * kRedStep + e;
+      float v = lds_sum<NW / 4>(r, kRedStep, NW / 4) * 16777216.f + lds_sum<NW / 4>(r + 64, kRedStep, NW / 4) * 1048576.f;
+      v += dpp_f32<0xB1>(v);
+      v += dpp_f32<0x4E>(v);
+      if (part == 0 && m < M) {
+        const float xs = lds_sum<NW / 2>(red + m * per_row * kRedStep + 128, kRedStep, per_row);
+        v -= zero_point * xs;
+        if (not_finite(xs)) v = elementwise_dot<4>(Wq + (size_t)n * rowb, X + (size_t)m * K, K, zero_point);
+        Y[(size_t)m * N + n] = static_cast<half_t>(v * (scalar_scale * scale_value(scale_now)));
+      }
+    }
+    if (!kOwnRed) __syncthreads();
   }
 }
 
@@ -874,37 +925,47 @@ bool launch_w8a16(const W8A16Args& a, hipStream_t s) {
   return true;
 }
 
-// Panel kernel (w4a16_x_kernel): where it measured ahead, us, the kernel it replaces / this one.
-//  * three and four rows, K up to 16384 (one pass): M=4 N=14336 K=5120 18.2 / 12.5, N=28672 K=2304 18.0 /
-//    12.0, N=12288 K=3072 10.5 / 7.6, N = K = 8192 12.7 / 11.2, N=4096 K=4096 6.0 / 4.7, K=14336 13.0 / 11.5;
-//    not with a second pass (N=4096 K=20480 15.4 / 19.3).  Narrow outputs leave its tiles on half the
-//    CUs: four rows still gain beyond 1024 columns (N=2048 K=8192 7.5 / 6.5), three are level (N = K = 2048 3.8 /
-//    3.8), N=1024 K=4096 M=3 4.0 / 4.2, K=16384 M=4 7.6 / 11.7.
-//  * two rows: the lanes-over-x kernel reads half the activations it does at four, so only for K up to
-//    4096 (N = K = 4096 4.9 / 4.4, N=28672 K=2304 13.9 / 11.3, N=12288 K=3072 7.5 / 6.8; N = K = 5120 6.4 / 7.7).
+// Panel kernel (w4a16_x_kernel): where it measured ahead of the lanes-over-x kernel and, for K <= 16384 and more
+// than 2048 columns, everywhere ahead of the row-load kernel (us, the other / this one, M = 2, 3, 4 where three pairs
+// stand).  It stages the whole panel whatever N is, so long rows need columns to spread that over; more activation
+// rows cost the lanes-over-x kernel as many more reads of x:
+//  * K <= 2048 always (N=512 K=512 2.6 / 2.5, 2.9 / 2.5, 3.3 / 2.5); K = 4096 N=1024 3.5 / 3.5, 4.0 / 3.6, 4.6 / 3.7,
+//    N=512 3.0 / 3.4, 3.4 / 3.5, 3.7 / 3.6;
+//  * K = 6144 N=1024 3.8 / 4.2, 4.5 / 4.4, 5.0 / 4.5, N=1536 4.3 / 4.3, 5.0 / 4.4, 5.4 / 4.5;
+//  * K = 8192 N=1024 4.1 / 4.9, 4.7 / 5.0, 5.2 / 5.3, N=1536 4.6 / 5.0, 5.4 / 5.1, 6.3 / 5.4, N=2048 5.1 / 5.1, N=3072
+//    5.9 / 5.6;
+//  * K = 12288 N=1024 4.9 / 6.5, 5.8 / 6.8, 6.6 / 7.1, N=1536 6.2 / 6.7, 7.4 / 6.9, 10.7 / 7.2, N=3072 7.6 / 7.2;
+//  * K = 16384 N=1536 6.6 / 7.9, 7.8 / 8.4, 10.9 / 8.7, N=2048 6.9 / 8.1, 8.2 / 8.5, N=3072 8.9 / 8.7, 10.9 / 9.1.
+// Against the row-load kernel N=4096 K=14336 M=4 13.0, N = K = 8192 12.7, N=5120 K=11008 16.9 (this one 9.9, 8.8, 10.4).
 static bool w4_panel(const W8A16Args& a) {
   if (a.K > 16384) return false;
-  if (a.M == 2) return a.N > 2048 && a.K <= 4096;
-  return a.N > 2048 || (a.M == 4 && a.N > 1024 && a.K <= 8192);
+  if (a.K <= 2048) return true;
+  if (a.K <= 4096) return a.M == 4 || a.N >= 1024;
+  if (a.K <= 6144) return a.N >= (a.M == 2 ? 1536 : 1024);
+  if (a.K <= 8192) return a.M == 2 ? a.N > 2048 : a.N >= 1536;
+  if (a.M == 2) return a.N >= 3072;
+  return a.M == 4 ? a.N >= 1536 : (a.K <= 12288 ? a.N >= 2048 : a.N > 2048);
 }
 static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
-#define FG_W4_X(KC, CB, NW)                                                                                     \
-  hipLaunchKernelGGL((w4a16_x_kernel<KC, CB, NW>), dim3(a.N / (16 * CB)), dim3(64 * NW), 0, s,                  \
+  // One workgroup a CU walks over up to two tiles, more where there are more tiles and LDS holds them: what it
+  // has in flight is one tile, 16 rows x K / 2 bytes, and shorter rows leave a CU idle (N=28672 K=2304 M=4 one / two a
+  // CU 11.9 / 8.9 us, K=1024 two / four 6.0 / 5.6), while with two tiles a second workgroup only stages the panel
+  // again (N=8192 K=3072 5.4 / 5.8).  KC: the smallest that holds K; four waves have enough to load up to K =
+  // 1024 (N=4096 3.1 / 2.7), sixteen share the largest panels (K=14336 10.8 / 10.4 with eight).
+  const int tiles = a.N / 16, cus = compute_units();
+#define FG_W4_X(KC, NW, MOST)                                                                                  \
+  hipLaunchKernelGGL((w4a16_x_kernel<KC, NW>),                                                                 \
+                     dim3(std::min(tiles, cus * std::min(MOST, (tiles + 2 * cus - 1) / (2 * cus)))), dim3(64 * NW), 0, s, \
                      static_cast<const uint8_t*>(a.Wq), static_cast<const half_t*>(a.x),                       \
                      static_cast<const half_t*>(a.scale), a.scalar_scale, a.zero_point, static_cast<half_t*>(a.y), \
                      a.M, a.N, a.K)
-  // 32 columns a workgroup stage the panel half as often, where N / 32 workgroups fill the CUs evenly
-  // (M=4 N=14336 K=4096 10.7 / 9.3; N=12288 K=3072, 384 workgroups, 7.6 / 8.6 the other way).  KC: the
-  // smallest that holds K; sixteen waves share the largest panels (K=14336 11.9 / 11.5 with eight).
-  const int t32 = a.N / 32;
-  const int cus = compute_units();
-  const bool wide = 8 * t32 >= 7 * ((t32 + cus - 1) / cus * cus);
-  if (a.K <= 2048) { if (wide) FG_W4_X(2048, 2, 8); else FG_W4_X(2048, 1, 8); }
-  else if (a.K <= 4096) { if (wide) FG_W4_X(4096, 2, 8); else FG_W4_X(4096, 1, 8); }
-  else if (a.K <= 6144) { if (wide) FG_W4_X(6144, 2, 8); else FG_W4_X(6144, 1, 8); }
-  else if (a.K <= 8192) { if (wide) FG_W4_X(8192, 2, 8); else FG_W4_X(8192, 1, 8); }
-  else if (a.K <= 12288) FG_W4_X(12288, 1, 16);
-  else FG_W4_X(16384, 1, 16);
+  if (a.K <= 1024) FG_W4_X(1024, 4, 4);
+  else if (a.K <= 2048) FG_W4_X(2048, 8, 2);
+  else if (a.K <= 4096) FG_W4_X(4096, 8, 2);
+  else if (a.K <= 6144) FG_W4_X(6144, 8, 1);
+  else if (a.K <= 8192) FG_W4_X(8192, 8, 1);
+  else if (a.K <= 12288) FG_W4_X(12288, 16, 1);
+  else FG_W4_X(16384, 16, 1);
 #undef FG_W4_X
 }
 

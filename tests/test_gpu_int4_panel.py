@@ -93,3 +93,21 @@ def test_smallest_and_largest_activations_are_exact(device, N, K, unit):
         want = ((m.numpy() @ W.T) * (unit * scalar)).astype(np.float32).astype(np.float16)
         assert (want != 0).mean() > 0.99
         assert (got == want).all(), (M, N, K)
+
+
+# tiles of 16 columns that a workgroup walks over: the last round partly filled, one to four workgroups a CU, every
+# panel size (the largest shares its LDS between the waves' strips and their sums)
+@pytest.mark.parametrize("N,K", [(33024, 128), (17408, 1024), (33024, 896), (8320, 1152), (12416, 2048), (8320, 2176),
+                                 (8320, 4224), (8320, 8192), (4224, 12160), (8320, 12416), (4224, 16384)])
+def test_many_tiles_a_workgroup_are_exact(device, N, K):
+    # |x| <= 8 and weights below 16: every sum is a whole number below 2^24, the scale a power of two
+    g = torch.Generator(device=device)
+    g.manual_seed(9950 + N + K)
+    Wd = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=device)
+    W = torch.stack((Wd & 15, Wd >> 4), dim=-1).flatten(1).double() - 8.0
+    for M in (2, 3, 4):
+        x = torch.randint(-8, 9, (M, K), generator=g, device=device).half()
+        scale = torch.pow(2.0, torch.randint(-3, 2, (N,), generator=g, device=device).float()).half()
+        got = _run(Wd, x, scale, 2.0 ** -6, 8.0, device)
+        want = (x.double() @ W.t() * scale.double() * 2.0 ** -6).half().cpu().numpy()
+        assert (got == want).all(), (M, N, K)
