@@ -12,6 +12,7 @@
 #include "fg_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace fg {
 
@@ -277,67 +278,125 @@ __global__ __launch_bounds__(256) void i8i8_kernel(const int8_t* __restrict__ Wq
   }
 }
 
-// Two to eight activation rows: as w4a16_x_kernel below, the activation panel in LDS and the weights from
-// memory straight into the operand of v_mfma_i32_16x16x64_i8 (16 bytes = 16 k of row j a lane), every
-// load of a wave's share in flight before the panel is staged.  XR = rows of the panel, 4 or 8; its
-// 16-byte pieces lie as [load][g][row].  Integer sums: exact in any order.  Launched with K <= KC.
+// Two to eight activation rows: as w4a16_x_kernel below, the activation panel in LDS, staged once a workgroup,
+// which then walks over column tiles of 16; the weights of a tile go from memory through registers and two KB of
+// wave-private LDS into the operand of v_mfma_i32_16x16x64_i8 (16 bytes = 16 k of row j a lane).  XR = rows of the
+// panel, 4 or 8; its 16-byte pieces lie as [64 k][g][row], the rows of a group permuted by its number (the threads
+// that stage it have consecutive k of one row).  Integer sums: exact in any order.  Launched with K <= KC.
+// What bounds it: the weights at what memory gives (N = K = 8192 M=8 12.4 us, 5.4 TB/s, a plain read 11.9), on
+// short calls launch, one memory latency for the panel and one for the weights (N=4096 K=2048 3.3).  Measured against
+// a panel kernel with loads in operand order (18 instead of 64 bytes a clock a CU, see w4a16_x_kernel) and one tile a
+// workgroup, us: M=8 N = K = 8192 15.9 / 12.4, N=14336 K=4096 16.6 / 11.3, N = K = 5120 11.4 / 7.3, N=4096 K=2048 3.7 /
+// 3.3; M=4, the v_dot4 kernel, N = K = 8192 13.5 / 12.3, N=8192 K=4096 8.7 / 7.3, N = K = 5120 7.5 / 7.2.
 template <int XR, int KC, int NW>
 __global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restrict__ Wq, const int8_t* __restrict__ Xq,
                                                          int32_t* __restrict__ out, int M, int N, int K) {
   typedef int int4_v __attribute__((ext_vector_type(4)));
-  constexpr int NT = 64 * NW;
-  constexpr int LOADS = KC / 64 / NW;         // weight loads a wave
-  constexpr int PIECES = XR * KC / 16 / NT;   // pieces of the panel a thread
-  static_assert(KC % (64 * NW) == 0 && XR * KC % (16 * NT) == 0, "whole loads and pieces");
+  constexpr int PAIRS = KC / 128 / NW;                // 16 rows x 128 bytes of weights: two loads a wave
+  // 1 KB of an activation row: one load a wave (fewer waves than rows: several rows a wave, one segment each)
+  constexpr bool kRows = NW < XR;
+  constexpr int SEGS = kRows ? XR / NW : (KC + 1023) / 1024 * XR / NW;
+  static_assert(KC % (128 * NW) == 0 && (KC % 1024 == 0 || KC < 1024) && (!kRows || KC <= 1024),
+                "whole pairs and segments");
+  constexpr int STRIP = 2048, RED = XR * 16;          // ints a wave hands over
+  constexpr bool kOwnRed = XR * KC + NW * (STRIP + 8 * RED) <= 160 * 1024;
   __shared__ u32x4 panel[XR * KC / 16];
-  __shared__ int red[NW][XR * 16];
+  __shared__ __attribute__((aligned(16))) unsigned char strips[NW * STRIP];
+  __shared__ int own_red[kOwnRed ? 2 * NW * RED : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int j = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int j = lane & 15, g = lane >> 4;             // operand order
+  const int lr = lane >> 3, lp = lane & 7;            // load order: row, 16-byte piece of its 128
   constexpr int kNonTemporal = 2;
-  const __amdgpu_buffer_rsrc_t wrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Wq + (size_t)n0 * K), 0, 16 * K, 0x00020000);
-  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Xq), 0, M * K, 0x00020000);
-  constexpr int kBeyond = 0x7ffffff0;         // past both descriptors: the load returns zeros
-  const int xm = tid % XR, xq = tid / XR;     // this thread's activation row and first 16-k piece of it
-  const int loads = K >> 6;
-  u32x4 x[PIECES], w[LOADS];
+  constexpr int kBeyond = 0x7ffffff0;                 // past the descriptors: the load returns zeros
   // activations first: loads return in order, and the panel must not wait for the weights
+  // waves that stage a row: NW / M
+  int per_row = kRows ? 1 : NW / XR;
+  if constexpr (XR == 4) per_row = M == 2 ? NW / 2 : (M == 3 ? NW / 3 : NW / 4);
+  else if constexpr (NW == 16) per_row = M == 5 ? 3 : 2;
+  const int xm = XR == 8 && NW <= 8 ? wave : wave / per_row, xs0 = kRows ? 0 : wave - xm * per_row;
+  u32x4 x[SEGS];
 #pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int q = xq + NT / XR * i;
-    const int off = (q * 16 < K && xm < M) ? xm * K + q * 16 : kBeyond;
-    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+  for (int i = 0; i < SEGS; ++i) {
+    const int row = xm + (kRows ? NW * i : 0), seg = xs0 + (kRows ? 0 : per_row * i);
+    const __amdgpu_buffer_rsrc_t xrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Xq + (size_t)row * K), 0, row < M ? K : 0, 0x00020000);
+    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, seg * 1024 + lane * 16, 0, 0));
   }
   __builtin_amdgcn_sched_barrier(0);
+  u32x4 w[PAIRS][2];
+  int w_off[PAIRS];
 #pragma unroll
-  for (int t = 0; t < LOADS; ++t) {
-    const int l = wave + NW * t;
-    const int off = l < loads ? j * K + l * 64 + g * 16 : kBeyond;
-    w[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, 0, kNonTemporal));
+  for (int t = 0; t < PAIRS; ++t) {
+    const int kb = (wave + NW * t) * 128 + lp * 16;
+    w_off[t] = kb < K ? lr * K + kb : kBeyond;
   }
-  __builtin_amdgcn_sched_barrier(0);
+  const int tiles = N >> 4;
+  auto load_pair = [&](int tile, int t) {
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(Wq + (size_t)tile * 16 * K), 0, tile < tiles ? 16 * K : 0, 0x00020000);
 #pragma unroll
-  for (int i = 0; i < PIECES; ++i) panel[(xq + NT / XR * i) * XR + xm] = x[i];
-  __syncthreads();
-  int4_v acc = {0, 0, 0, 0};
+    for (int h = 0; h < 2; ++h)
+      w[t][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              wrs, w_off[t] == kBeyond ? kBeyond : w_off[t] + 8 * h * K, 0, kNonTemporal));
+  };
+  int tile = blockIdx.x;
 #pragma unroll
-  for (int t = 0; t < LOADS; ++t)             // (past the end of K: zero weights on a zero panel)
-    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-        __builtin_bit_cast(int4_v, panel[((wave + NW * t) * 4 + g) * XR + j % XR]), __builtin_bit_cast(int4_v, w[t]),
-        acc, 0, 0, 0);
-  // acc[r]: row 4g + r, column j
-  if (4 * g < XR) {
+  for (int t = 0; t < PAIRS; ++t) {
+    load_pair(tile, t);
+    __builtin_amdgcn_sched_barrier(0);                // in this order: they are waited for one after the other
+  }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[wave][(4 * g + r) * 16 + j] = acc[r];
+  for (int i = 0; i < SEGS; ++i) {
+    const int row = xm + (kRows ? NW * i : 0), seg = xs0 + (kRows ? 0 : per_row * i);
+    const int q = seg * 64 + lane;                    // 16-k piece
+    asm volatile("" : "+v"(x[i]));                    // (or the load sinks below the weights', to its only use)
+    if (row < M && q < KC / 16) panel[q * XR + (row ^ ((q >> 2) & (XR - 1)))] = x[i];
   }
   __syncthreads();
-  if (tid < XR * 16) {
-    int sum = 0;
+
+  unsigned char* const strip = strips + wave * STRIP;
+  for (int parity = 0; tile < tiles; tile += gridDim.x, parity ^= 1) {
+    int4_v acc = {0, 0, 0, 0};
+    const int next = tile + (int)gridDim.x;
+    auto walk = [&](auto more) {
 #pragma unroll
-    for (int v = 0; v < NW; ++v) sum += red[v][tid];
-    if ((tid >> 4) < M) out[(size_t)(tid >> 4) * N + n0 + (tid & 15)] = sum;
+      for (int t = 0; t < PAIRS; ++t) {
+        const int pair = wave + NW * t;
+        u32x4 xv[2];                                  // the panel's operands do not wait for the weights
+#pragma unroll
+        for (int u = 0; u < 2; ++u) xv[u] = panel[((pair * 2 + u) * 4 + g) * XR + ((j ^ (pair * 2 + u)) & (XR - 1))];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4*>(strip + h * 1024 + lr * 128 + 16 * (lp ^ lr)) = w[t][h];
+        wave_lds_sync();
+        if constexpr (more) load_pair(next, t);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {                 // (past the end of K: zero weights)
+          const u32x4 wv = *reinterpret_cast<const u32x4*>(strip + j * 128 + 16 * ((4 * u + g) ^ (j & 7)));
+          acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(int4_v, xv[u]), __builtin_bit_cast(int4_v, wv),
+                                                      acc, 0, 0, 0);
+        }
+        wave_lds_sync();
+      }
+    };
+    if (next < tiles) walk(std::true_type{});
+    else walk(std::false_type{});
+    // acc[r]: row 4g + r, column j
+    int* const red = kOwnRed ? own_red + parity * NW * RED : reinterpret_cast<int*>(strips);
+    constexpr int kRedStep = kOwnRed ? RED : STRIP / 4;
+    if (4 * g < XR) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave * kRedStep + (4 * g + r) * 16 + j] = acc[r];
+    }
+    __syncthreads();
+    if (tid < XR * 16) {
+      int sum = 0;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) sum += red[v * kRedStep + tid];
+      if ((tid >> 4) < M) out[(size_t)(tid >> 4) * N + tile * 16 + (tid & 15)] = sum;
+    }
+    if (!kOwnRed) __syncthreads();
   }
 }
 
@@ -946,16 +1005,19 @@ static bool w4_panel(const W8A16Args& a) {
   if (a.M == 2) return a.N >= 3072;
   return a.M == 4 ? a.N >= 1536 : (a.K <= 12288 ? a.N >= 2048 : a.N > 2048);
 }
+// Workgroups of a panel kernel: one a CU walks over up to `each` tiles, more where there are more tiles and LDS holds
+// them (`most`).  What a workgroup has in flight is one tile, 16 weight rows, and short rows leave a CU idle (int4 M=4
+// N=28672 K=2304 one / two a CU 11.9 / 8.9 us, K=1024 two / four 6.0 / 5.6), while for two tiles of longer rows a second
+// workgroup only stages the panel again (N=8192 K=3072 5.4 / 5.8, K=2048 3.9 / 4.2; K=1024 the other way, 3.4 / 3.3).
+static int panel_grid(int tiles, int cus, int each, int most) {
+  return std::min(tiles, cus * std::min(most, (tiles + each * cus - 1) / (each * cus)));
+}
 static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
-  // One workgroup a CU walks over up to two tiles, more where there are more tiles and LDS holds them: what it
-  // has in flight is one tile, 16 rows x K / 2 bytes, and shorter rows leave a CU idle (N=28672 K=2304 M=4 one / two a
-  // CU 11.9 / 8.9 us, K=1024 two / four 6.0 / 5.6), while with two tiles a second workgroup only stages the panel
-  // again (N=8192 K=3072 5.4 / 5.8).  KC: the smallest that holds K; four waves have enough to load up to K =
-  // 1024 (N=4096 3.1 / 2.7), sixteen share the largest panels (K=14336 10.8 / 10.4 with eight).
+  // KC: the smallest that holds K; four waves have enough to load up to K = 1024 (N=4096 3.1 / 2.7), sixteen share the
+  // largest panels (K=14336 10.8 / 10.4 with eight).
   const int tiles = a.N / 16, cus = compute_units();
 #define FG_W4_X(KC, NW, MOST)                                                                                  \
-  hipLaunchKernelGGL((w4a16_x_kernel<KC, NW>),                                                                 \
-                     dim3(std::min(tiles, cus * std::min(MOST, (tiles + 2 * cus - 1) / (2 * cus)))), dim3(64 * NW), 0, s, \
+  hipLaunchKernelGGL((w4a16_x_kernel<KC, NW>), dim3(panel_grid(tiles, cus, KC <= 1024 ? 1 : 2, MOST)), dim3(64 * NW), 0, s, \
                      static_cast<const uint8_t*>(a.Wq), static_cast<const half_t*>(a.x),                       \
                      static_cast<const half_t*>(a.scale), a.scalar_scale, a.zero_point, static_cast<half_t*>(a.y), \
                      a.M, a.N, a.K)
@@ -1003,18 +1065,16 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
   // wave, and three or four waves, whichever leaves fewer of the last step's waves without a piece; the
   // other, below, eight rows (four for narrow outputs), two pieces a wave, four waves.  One after the other in
   // a replayed graph, us, the second form / the first:
-  //  * two rows: the first throughout (N = K = 5120 7.2 / 6.5, N = K = 8192 12.6 / 12.1, N=28672 K=8192 36.5 /
-  //    34.7, K=12288 52.0 / 51.7), three rows too (8.2 / 7.3, 13.5 / 13.2, 37.0 / 37.1, 53.4 / 54.9);
-  //  * four rows: the first (N = K = 5120 8.4 / 7.5, N=14336 K=4096 14.6 / 12.8, N=12288 K=8704 21.8 / 20.9,
-  //    N=16384 K=11008 33.6 / 32.6) but for eight and twelve pieces against wide outputs, where the second's
-  //    waves all have as many (N=8192 K=7936 13.7 / 14.1, N=28672 K=7936 36.0 / 39.5, N = K = 8192 13.9 / 14.1;
-  //    N = K = 12288 26.0 / 28.2, N=28672 K=11520 52.0 / 55.9; N=5120 K=8192 11.1 / 10.2, N=11008 K=12288
+  //  * two and three rows: the first throughout (M=2 N = K = 8192 12.6 / 12.1, N=28672 K=8192 36.5 / 34.7, K=12288 52.0 /
+  //    51.7, M=3 53.4 / 54.9);
+  //  * four rows: the first (N=16384 K=11008 33.6 / 32.6) but for twelve pieces against wide outputs, where the
+  //    second's waves all have as many (N = K = 12288 26.0 / 28.2, N=28672 K=11520 52.0 / 55.9; N=11008 K=12288
   //    25.0 / 25.2);
-  //  * narrow outputs keep the second, their workgroups do not fill the chip (N=2048 K=6144 M=4 5.3 /
-  //    5.4, K=14336 7.9 / 8.5), and so do the longest rows (N=4096 K=14336 M=4 12.8 / 13.0).
+  //  * narrow outputs keep the second, their workgroups do not fill the chip (N=2048 K=14336 M=4 7.9 / 8.5), and so
+  //    do the longest rows (N=4096 K=14336 M=4 12.8 / 13.0).
   if (MB == 2 || MB == 4) {
     const int pieces = (K / 16 + 63) / 64;
-    const bool full_steps = M == 4 && pieces >= 8 && pieces % 4 == 0 && N >= 1024 * pieces;
+    const bool full_steps = M == 4 && pieces == 12 && N >= 1024 * pieces;
     if (N > 2048 && pieces <= 12 && !full_steps) {
       const int waves = pieces <= 4 ? pieces : ((pieces + 2) / 3 * 3 < (pieces + 3) / 4 * 4 ? 3 : 4);
       hipLaunchKernelGGL((i8i8_kernel<MB, 4, 1>), dim3(N / 4), dim3(64 * waves), 0, s, W, X, acc, M, N, K);
@@ -1033,28 +1093,25 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
   }
 }
 
-// Panel kernel (i8i8_x_kernel): where it measured ahead, us, the v_dot4 kernel / this one.
-//  * five to eight rows, which cost the v_dot4 kernel a register tile per row: M=8 N=14336 K=4096 22.9 / 16.6,
-//    K=5120 24.5 / 20.7; N = K = 8192 19.1 / 16.0, N = K = 4096 8.8 / 5.9; N=4096 K=14336 16.7 / 14.9.  Not
-//    narrow outputs with long rows (N=2048 K=8192 7.7 / 8.2, K=4096 5.9 / 5.1; N=1024 K=4096 4.7 / 5.0), and
-//    not tiles that leave a third of the CUs' second round idle (N = K = 5120, 320 tiles, M=5 10.5 / 10.6).
-//  * two to four rows: short rows, the shorter the wider the output (K=1024 M=4 N=11008 5.1 / 4.7, N=28672
-//    8.1 / 8.0; K=2048 N=2048 4.0 / 3.3, N=8192 5.5 / 5.2, N=16384 8.5 / 8.4, N=28672 12.0 / 12.9; M=2 K=1024
-//    N=11008 4.4 / 4.3, N=14336 4.9 / 5.3, K=2048 N=8192 5.1 / 4.9, N=11008 6.0 / 6.4);
-//  * three and four rows with one workgroup on every CU or nearly (M=4 K=4096 N=3072 5.3 / 4.9, N=4096 6.0 /
-//    5.2; M=3 5.2 / 4.9, 5.8 / 5.2), on every CU up to K = 6144 (N=4096 M=4 7.2 / 6.9, M=3 6.8 / 6.8; N=3072 6.0 /
-//    6.6).  A second one a CU, or a longer row, and 1 KB of a row a load beats 16 rows x 64 bytes (K=4096 M=4
-//    N=8192 8.8 / 8.8, N=12288 11.5 / 12.1, N=16384 14.1 / 15.2, N=4224 6.2 / 7.5; N = K = 5120 7.5 / 10.4).
+// Panel kernel (i8i8_x_kernel): where it measured ahead, us, the v_dot4 kernel (or an earlier panel kernel, with loads
+// in operand order and one tile a workgroup) / this one.  It stages the whole panel whatever N is, so long rows need
+// columns to spread that over:
+//  * five rows and more: N=1024 K=4096 M=8 4.6 / 3.8, K=6144 5.1 / 4.8, K=8192 5.5 / 6.0; N=1536 K=8192 7.4 / 6.2, K=12288
+//    9.6 / 8.6; N=2048 K=14336 M=5 9.4 / 10.4, N=3072 M=8 14.4 / 11.7; N = K = 5120 11.4 / 7.3, N = K = 8192 15.9 / 12.4,
+//    N=14336 K=4096 16.6 / 11.3;
+//  * four: N=1024 K=4096 3.7 / 3.4, K=5120 4.0 / 4.4; N=1536 K=8192 5.7 / 5.6; N=2048 K=9216 6.9 / 7.3, N=3072 7.7 / 7.9; N =
+//    K = 5120 7.5 / 7.2, N=4096 K=8192 8.6 / 7.5, N=14336 K=4096 12.4 / 11.2, N = K = 8192 13.5 / 12.3; three, less: N=2048
+//    K=8192 6.0 / 5.8, N=9216 K=5120 10.0 / 10.3, N=5120 K=8192 9.4 / 9.6;
+//  * two, for which the v_dot4 kernel reads few activations: K <= 2048 (N=28672 10.9 / 10.3, N=2048 3.3 / 2.9), to K = 4096
+//    with one tile a CU at most (N=4096 5.2 / 4.7), to 6144 where one or two tiles a CU come out even (N=8192 9.6 / 9.0,
+//    N=7168 8.8 / 8.2; N=5120 7.3 / 7.7, N=9216 10.5 / 11.3).
 static bool i8_panel(int M, int N, int K) {
-  if (M < 2 || N < 2048 || K > 16384) return false;
-  const int tiles = N / 16, cus = compute_units();
-  if (M >= 5) {
-    const bool even = 10 * tiles >= 7 * ((tiles + cus - 1) / cus * cus);
-    return K <= 4096 || (N > 2048 && even);
-  }
-  if (M == 2) return K <= 512 || (K <= 2048 && N <= 8192);
-  if (K <= 1536 || (K <= 2048 && N <= 16384)) return true;
-  return tiles <= cus && 4 * tiles >= 3 * cus && K <= (tiles == cus ? 6144 : 4096);
+  if (M < 2 || K > 16384) return false;
+  if (M >= 5) return K <= 4096 || N >= (K <= 6144 ? 1024 : (K <= 12288 ? 1536 : 2176));
+  if (K <= 2048) return true;
+  if (M >= 3) return K <= 4096 ? N >= (M == 4 ? 512 : 1024) : (K <= 8192 && N >= (M == 4 ? 1536 : 2048));
+  const int tiles = N / 16, cus = compute_units(), rounds = (tiles + cus - 1) / cus;
+  return (K <= 4096 && rounds == 1 && N >= 2048) || (K <= 6144 && rounds <= 2 && 8 * tiles >= 7 * rounds * cus);
 }
 
 bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N, int K,
@@ -1063,19 +1120,26 @@ bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N,
   if (i8_panel(M, N, K)) {
     auto* W = static_cast<const int8_t*>(Wq);
     auto* X = static_cast<const int8_t*>(xq);
-#define FG_I8_X(XR, KC, NW) \
-  hipLaunchKernelGGL((i8i8_x_kernel<XR, KC, NW>), dim3(N / 16), dim3(64 * NW), 0, s, W, X, acc, M, N, K)
-    if (M <= 4) {  // up to K = 6144, see i8_panel
-      if (K <= 2048) FG_I8_X(4, 2048, 8);
-      else if (K <= 4096) FG_I8_X(4, 4096, 8);
-      else if (K <= 6144) FG_I8_X(4, 6144, 8);
-      else return false;
-    } else if (K <= 2048) FG_I8_X(8, 2048, 8);
-    else if (K <= 4096) FG_I8_X(8, 4096, 8);
-    else if (K <= 6144) FG_I8_X(8, 6144, 8);
-    else if (K <= 8192) FG_I8_X(8, 8192, 8);
-    else if (K <= 12288) FG_I8_X(8, 12288, 16);
-    else FG_I8_X(8, 16384, 16);
+    // Workgroups a CU as in launch_w4_panel.
+    const int tiles = N / 16, cus = compute_units();
+#define FG_I8_X(XR, KC, NW, MOST)                                                                    \
+  hipLaunchKernelGGL((i8i8_x_kernel<XR, KC, NW>), dim3(panel_grid(tiles, cus, KC <= 1024 ? 1 : 2, MOST)), \
+                     dim3(64 * NW), 0, s, W, X, acc, M, N, K)
+    if (M <= 4) {
+      if (K <= 512) FG_I8_X(4, 512, 4, 4);
+      else if (K <= 1024) FG_I8_X(4, 1024, 4, 4);
+      else if (K <= 2048) FG_I8_X(4, 2048, 8, 3);
+      else if (K <= 4096) FG_I8_X(4, 4096, 8, 2);
+      else if (K <= 6144) FG_I8_X(4, 6144, 8, 2);
+      else FG_I8_X(4, 8192, 8, 2);              // (longer rows: see i8_panel)
+    } else if (K <= 512) FG_I8_X(8, 512, 4, 4);
+    else if (K <= 1024) FG_I8_X(8, 1024, 8, 3);
+    else if (K <= 2048) FG_I8_X(8, 2048, 8, 2);
+    else if (K <= 4096) FG_I8_X(8, 4096, 8, 2);
+    else if (K <= 6144) FG_I8_X(8, 6144, 8, 1);
+    else if (K <= 8192) FG_I8_X(8, 8192, 8, 1);
+    else if (K <= 12288) FG_I8_X(8, 12288, 16, 1);
+    else FG_I8_X(8, 16384, 16, 1);
 #undef FG_I8_X
   } else if (M == 1) {
     i8i8_go<1>(Wq, xq, acc, M, N, K, s);

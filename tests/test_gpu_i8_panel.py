@@ -1,8 +1,7 @@
 """int8 x int8 products of two to eight activation rows, which the kernel that holds them in LDS as one panel
-and the v_dot4 kernel share between them: K at and beside the panel sizes (five rows and more run the
-panel there, two to four up to K = 2048, three and four against 4096 outputs up to 6144, the v_dot4
-kernel the rest), sizes on both sides of each line of the rule, whole int8 range, exact to the bit;
-nothing is written behind the result."""
+and the v_dot4 kernel share between them: K at and beside the panel sizes, sizes on both sides of each line
+of the rule, workgroups that walk over several column tiles, whole int8 range, exact to the bit; nothing is
+written behind the result."""
 import pytest
 import torch
 
@@ -55,6 +54,26 @@ def test_lines_of_the_rule_are_exact(device, N, K):
     W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)
     W64 = W.double().t()
     for M in (2, 3, 4):
+        x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=device)
+        acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
+        assert capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr()) == capi.FG_OK
+        assert torch.equal(acc[:M], (x.double() @ W64).round().int()), (M, N, K)
+        assert bool((acc[M] == -3).all())
+
+
+# column tiles that a workgroup walks over (the last round partly filled; one to four workgroups a CU), and both sides
+# of the rule's lines for five rows and more, for narrow outputs and for two rows
+@pytest.mark.parametrize("N,K", [(128, 128), (33024, 256), (33024, 512), (17408, 640), (17408, 1024), (14464, 1152),
+                                 (8320, 2048), (8320, 2176), (12416, 4096), (4224, 4224), (8320, 5248), (8320, 8064),
+                                 (512, 4096), (1024, 4096), (1024, 4224), (896, 6144), (1024, 6272), (1536, 8192),
+                                 (1408, 8192), (1536, 8320), (2048, 12416), (2176, 12416), (3584, 5120), (3456, 5120),
+                                 (7168, 6144), (4224, 8192), (4224, 12288), (4224, 16384)])
+def test_many_tiles_and_narrow_outputs_are_exact(device, N, K):
+    g = torch.Generator(device=device)
+    g.manual_seed(9850 + N + K)
+    W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)
+    W64 = W.double().t()
+    for M in range(2, 9):
         x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=device)
         acc = torch.full((M + 1, N), -3, dtype=torch.int32, device=device)
         assert capi.lib().fg_gemv_i8i8_i32(ptr(W), ptr(x), ptr(acc), M, N, K, stream_ptr()) == capi.FG_OK
