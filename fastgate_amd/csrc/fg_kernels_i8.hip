@@ -863,6 +863,157 @@ __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restr
 }
 
 // ---------------------------------------------------------------------------------------
+// w8a16, two to sixteen activation rows whose panel fits LDS: as w4a16_x_kernel above.  A workgroup stages the panel
+// once, XR rows (4, 8 or 16; M <= XR) of K fp16 in operand order, and walks over 16-column tiles with only weights left
+// to load.  The row-load kernel reads the activations again for every tile, and a CU takes HBM and L2 lines in the order
+// it asked for them, some 50 GB/s together: with 16 rows the activations are two thirds of its bytes.  Lane (j, g) takes
+// 16 bytes = 16 k of row j, the operands of two MFMAs; the panel's 16-byte pieces lie as [64 k][lower, upper 8 k of a
+// lane's 16][g][row], the rows of a piece permuted by its number against bank conflicts.  With few waves (NW < XR) a wave
+// stages several rows.  Bound by HBM for outputs of several tiles a CU (N=128256 K=2048, sixteen rows 44.2 us, 5.9 TB/s;
+// row-load kernel 86.7), by the panel's way through L2 and the first weights' latency for one.  us, before / this one:
+//   M=16  4096 x 4096 7.4 / 6.4   8192 x 2048 7.1 / 5.6   14336 x 4096 17.1 / 12.8   28672 x 1024 14.8 / 7.5
+//   M=8   5120 x 5120 10.4 / 8.5  11008 x 4096 14.2 / 10.1   8192 x 8192 15.1 / 14.3   14336 x 4096 13.0 / 12.2
+//   M=4   4096 x 4096 6.1 / 5.4   8192 x 2048 5.8 / 4.9   28672 x 2048 13.0 / 10.9   M=2 4096 x 2048 4.3 / 3.6
+// Launched with K <= KC.
+// ---------------------------------------------------------------------------------------
+template <int XR, int KC, int NW>
+__global__ __launch_bounds__(64 * NW) void w8a16_x_kernel(const int8_t* __restrict__ Wq, const half_t* __restrict__ X,
+                                                          const half_t* __restrict__ scale, float scalar_scale,
+                                                          float zero_point, half_t* __restrict__ Y, int M, int N, int K) {
+  constexpr int PAIRS = KC / 128 / NW;                // 16 rows x 128 bytes of weights: two loads a wave
+  constexpr int SEGS = KC / 512 * XR / NW;            // 1 KB of an activation row: one load a wave
+  static_assert(KC % (128 * NW) == 0 && KC % 512 == 0 && KC / 512 * XR % NW == 0, "whole pairs and segments");
+  constexpr int ROWS = NW < XR ? XR / NW : 1;         // rows a wave stages; or NW / M waves stage a row
+  constexpr int STRIP = 2048, RED = XR * 16 + ROWS;   // floats a wave hands over: sums, and its parts of sums of x
+  constexpr bool kOwnRed = XR * KC * 2 + NW * (STRIP + 8 * RED) <= 160 * 1024 - 64;
+  __shared__ u32x4 panel[XR * KC / 8];
+  __shared__ __attribute__((aligned(16))) unsigned char strips[NW * STRIP];
+  __shared__ float own_red[kOwnRed ? 2 * NW * RED : 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, g = lane >> 4;             // operand order
+  const int lr = lane >> 3, lp = lane & 7;            // load order: row, 16-byte piece of its 128
+  constexpr int kNonTemporal = 2;
+  constexpr int kBeyond = 0x7ffffff0;                 // past the descriptors: the load returns zeros
+  constexpr int kShift = XR == 16 ? 0 : (XR == 8 ? 1 : 2);
+  auto place = [&](int piece, int row) { return piece * XR + (row ^ ((piece >> kShift) & (XR - 1))); };
+  // activations first: loads return in order, and the panel must not wait for the weights
+  int per_row = NW < XR ? 1 : NW / XR;                // waves that stage a row: NW / M
+  if constexpr (XR == 4) per_row = M == 2 ? NW / 2 : (M == 3 ? NW / 3 : NW / 4);
+  else if constexpr (XR == 8 && NW == 16) per_row = M == 5 ? 3 : 2;
+  const int xm = NW < XR ? wave * ROWS : wave / per_row, xs0 = wave - wave / per_row * per_row;
+  u32x4 x[SEGS];
+#pragma unroll
+  for (int i = 0; i < SEGS; ++i) {
+    const int m = xm + i % ROWS;
+    const __amdgpu_buffer_rsrc_t xrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(X + (size_t)m * K), 0, m < M ? K * 2 : 0, 0x00020000);
+    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                         xrs, (xs0 + per_row * (i / ROWS)) * 1024 + lane * 16, 0, 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int tiles = N >> 4;
+  int tile = blockIdx.x;
+  // scale of the output this thread writes, ahead of the tile's weights
+  uint32_t scale_raw = scale_fetch(scale, tile * 16 + j, tid < XR * 16);
+  u32x4 w[PAIRS][2];
+  int w_off[PAIRS];
+#pragma unroll
+  for (int t = 0; t < PAIRS; ++t) {
+    const int kb = (wave + NW * t) * 128 + lp * 16;
+    w_off[t] = kb < K ? lr * K + kb : kBeyond;
+  }
+  auto load_pair = [&](int of, int t) {
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(Wq + (size_t)of * 16 * K), 0, of < tiles ? 16 * K : 0, 0x00020000);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[t][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              wrs, w_off[t] == kBeyond ? kBeyond : w_off[t] + 8 * h * K, 0, kNonTemporal));
+  };
+#pragma unroll
+  for (int t = 0; t < PAIRS; ++t) {
+    load_pair(tile, t);
+    __builtin_amdgcn_sched_barrier(0);                // in this order: they are waited for one after the other
+  }
+  const half2_t ones = {static_cast<half_t>(1.f), static_cast<half_t>(1.f)};
+  float xsum[ROWS] = {};
+#pragma unroll
+  for (int i = 0; i < SEGS; ++i) {
+    const int m = xm + i % ROWS, k8 = (xs0 + per_row * (i / ROWS)) * 64 + lane;   // row, 8-k group
+    asm volatile("" : "+v"(x[i]));                    // (or the load sinks below the weights', to its only use)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) xsum[i % ROWS] = __builtin_amdgcn_fdot2(as_half2(x[i][c]), ones, xsum[i % ROWS], false);
+    if (m < M && k8 < KC / 8) panel[place((k8 >> 3) * 8 + (k8 & 1) * 4 + ((k8 >> 1) & 3), m)] = x[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) xsum[i] = wave_sum(xsum[i]);
+
+  unsigned char* const strip = strips + wave * STRIP;
+  for (int parity = 0; tile < tiles; tile += gridDim.x, parity ^= 1) {
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const int next = tile + (int)gridDim.x;
+    const uint32_t scale_now = scale_raw;
+    scale_raw = scale_fetch(scale, next * 16 + j, tid < XR * 16 && next < tiles);
+    auto walk = [&](auto more) {
+#pragma unroll
+      for (int t = 0; t < PAIRS; ++t) {
+        const int pair = wave + NW * t;
+        u32x4 xv[2][2];                               // the panel's operands do not wait for the weights
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) xv[u][h] = panel[place(((pair * 2 + u) * 2 + h) * 4 + g, j & (XR - 1))];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4*>(strip + h * 1024 + lr * 128 + 16 * (lp ^ lr)) = w[t][h];
+        wave_lds_sync();
+        if constexpr (more) load_pair(next, t);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {                 // (past the end of K: zero activations)
+          const u32x4 wv = *reinterpret_cast<const u32x4*>(strip + j * 128 + 16 * ((4 * u + g) ^ (j & 7)));
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            // bytes as fp16 subnormals, (w + 128) 2^-24; the 128 leaves with the zero point
+            const uint32_t t0 = wv[2 * h] ^ 0x80808080u, t1 = wv[2 * h + 1] ^ 0x80808080u;
+            const u32x4 wb = {__builtin_amdgcn_perm(0u, t0, 0x04010400u), __builtin_amdgcn_perm(0u, t0, 0x04030402u),
+                              __builtin_amdgcn_perm(0u, t1, 0x04010400u), __builtin_amdgcn_perm(0u, t1, 0x04030402u)};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(xv[u][h]), as_half8(wb), acc, 0, 0, 0);
+          }
+        }
+        wave_lds_sync();
+      }
+    };
+    if (NW == 8 && next >= tiles) walk(std::false_type{});
+    else walk(std::true_type{});
+    // acc[r]: row 4g + r, column j
+    float* const red = kOwnRed ? own_red + parity * NW * RED : reinterpret_cast<float*>(strips);
+    constexpr int kRedStep = kOwnRed ? RED : STRIP / 4;
+    if (4 * g < XR) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave * kRedStep + (4 * g + r) * 16 + j] = acc[r];
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) red[wave * kRedStep + XR * 16 + i] = xsum[i];
+    }
+    __syncthreads();
+    if (tid < XR * 16 && (tid >> 4) < M) {
+      const int m = tid >> 4, n = tile * 16 + j;
+      const float sum = lds_sum<NW>(red + tid, kRedStep, NW);
+      const float* const xr = red + (m / ROWS) * per_row * kRedStep + XR * 16 + m % ROWS;
+      const float xs = lds_sum<(NW < XR ? 1 : XR == 4 ? NW / 2 : NW / XR + 1)>(xr, kRedStep, per_row);
+      float v = sum * 16777216.f - (zero_point + 128.f) * xs;
+      if (not_finite(xs))
+        v = elementwise_dot<8>(reinterpret_cast<const uint8_t*>(Wq) + (size_t)n * K, X + (size_t)m * K, K, zero_point);
+      Y[(size_t)m * N + n] = static_cast<half_t>(v * (scalar_scale * scale_value(scale_now)));
+    }
+    if (!kOwnRed) __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Host launchers.  The integer-dot kernel, beyond what i8i8_go says of two to four rows: rows per workgroup
 // 8 when that still yields >= 512 workgroups, else 4; waves as many (<= 4) as the row has 1 KB pieces.
 // ---------------------------------------------------------------------------------------
@@ -908,6 +1059,91 @@ static void launch_wq_m1(const W8A16Args& a, hipStream_t s) {
 #undef FG_WQ_M1
 }
 
+// Workgroups of a panel kernel: one a CU walks over up to `each` tiles, more where there are more tiles and LDS holds
+// them (`most`).  What a workgroup has in flight is one tile, 16 weight rows, and short rows leave a CU idle (int4 M=4
+// N=28672 K=2304 one / two a CU 11.9 / 8.9 us, K=1024 two / four 6.0 / 5.6), while for two tiles of longer rows a second
+// workgroup only stages the panel again (N=8192 K=3072 5.4 / 5.8, K=2048 3.9 / 4.2; K=1024 the other way, 3.4 / 3.3).
+static int panel_grid(int tiles, int cus, int each, int most) {
+  return std::min(tiles, cus * std::min(most, (tiles + each * cus - 1) / (each * cus)));
+}
+// Panel kernel (w8a16_x_kernel): where it measured ahead of the row-load and lanes-over-x kernels (us, the better of
+// those / this one):
+//  * nine rows and more, wherever the panel fits: N=512 K=128 3.1 / 2.6, N=4096 K=4096 7.4 / 6.4, N=28672 K=2048 23.5 /
+//    11.8, N=14336 K=4096 17.1 / 12.8;
+//  * five to eight: N = K = 512 3.1 / 2.5, N=5120 K=5120 10.4 / 8.5, N = K = 8192 14.9 / 14.1 -- except one tile of long
+//    rows on nearly every CU, which waits for the panel with little to spread it over (N=4096 K=6400 8.6 / 8.9, K=8192
+//    9.6 / 9.8; N=3584 K=7168 8.8 / 8.6);
+//  * two to four, for which the others read few activations: K <= 2048 (N=28672 K=1536 11.5 / 8.6, N=512 K=1792 3.3 /
+//    2.9), and from there outputs wide enough to pay for the panel.  Four: N=1024 K=3072 4.0 / 3.7, N=512 K=2560 3.5 /
+//    3.6; N=1536 K=4608 5.7 / 5.2, N=1024 K=4096 4.4 / 4.5.  Three: N=1536 K=2560 4.0 / 3.7, N=512 3.3 / 3.6; N=2048
+//    K=4096 4.9 / 4.7, N=1536 4.4 / 4.6; N=3072 K=8192 8.5 / 7.8, N=1536 6.6 / 7.0.  Two: N=2048 K=3072 3.9 / 3.8; N=4096
+//    K=4096 5.9 / 5.4, N=2048 4.3 / 4.6, N=14336 12.5 / 12.1, N=5120 6.5 / 6.9 (the second round a quarter full);
+//    N=11008 K=8192 18.0 / 16.4, N=3072 7.4 / 7.7;
+//  * not K > 6144 where 16-column tiles come out even, N = 8192 K=8192 four rows 12.9 / 13.2, two 11.5 / 11.9 at K=7168.
+static bool w8_panel(const W8A16Args& a) {
+  const int tiles = a.N / 16, cus = compute_units(), rounds = (tiles + cus - 1) / cus;
+  if (a.M >= 9) return a.K <= 4096;
+  if (a.M >= 5) return a.K <= 6144 || (a.K <= 8192 && (8 * tiles <= 7 * cus || rounds > 1));
+  if (a.K <= 2048) return true;
+  if (a.K > 8192 || (a.K > 6144 && tiles == rounds * cus)) return false;
+  if (a.M == 4) return 8 * tiles >= (a.K <= 3072 ? 2 : 3) * cus;
+  if (a.M == 3) return 4 * tiles >= (a.K <= 3072 ? 1 : (a.K <= 6144 ? 2 : 3)) * cus;
+  if (a.K <= 3072 && rounds <= 2) return 2 * tiles >= cus;
+  if (rounds == 1) return a.K <= 6144 && 8 * tiles >= 5 * cus;
+  return 4 * tiles > 3 * rounds * cus;
+}
+static void launch_w8_panel(const W8A16Args& a, hipStream_t s) {
+  // KC: the smallest that holds K.  Few waves with several pairs each where that keeps loads enough in flight (us, eight
+  // rows, one way / the other: N=8192 K=2560 eight waves of three pairs 6.7 / four of five 5.7; K=5120 sixteen waves 10.6
+  // / eight of five 10.0; K=7168 12.4 sixteen / 11.5 eight of seven); more where one tile is all a workgroup does (N=1024
+  // K=2048 four / eight 3.7 / 3.5), and sixteen of two pairs at K = 4096 (N=8192 8.7 / 8.1 with eight of four).
+  const int tiles = a.N / 16, cus = compute_units();
+  const bool many = tiles > cus;
+#define FG_W8_X(XR, KC, NW, MOST)                                                                                  \
+  hipLaunchKernelGGL((w8a16_x_kernel<XR, KC, NW>), dim3(panel_grid(tiles, cus, KC <= 512 ? 1 : 2, MOST)), dim3(64 * NW), \
+                     0, s, static_cast<const int8_t*>(a.Wq), static_cast<const half_t*>(a.x),                      \
+                     static_cast<const half_t*>(a.scale), a.scalar_scale, a.zero_point, static_cast<half_t*>(a.y), \
+                     a.M, a.N, a.K)
+  if (a.M <= 4) {
+    if (a.K <= 512) FG_W8_X(4, 512, 4, 4);
+    else if (a.K <= 1024) FG_W8_X(4, 1024, 8, 4);
+    else if (a.K <= 1536) FG_W8_X(4, 1536, 4, 4);
+    else if (a.K <= 2048) FG_W8_X(4, 2048, 8, 2);
+    else if (a.K <= 2560) FG_W8_X(4, 2560, 4, 3);
+    else if (a.K <= 3072) FG_W8_X(4, 3072, 8, 2);
+    else if (a.K <= 4096 && !many) FG_W8_X(4, 4096, 8, 1);
+    else if (a.K <= 4096) FG_W8_X(4, 4096, 16, 1);
+    else if (a.K <= 5120) FG_W8_X(4, 5120, 8, 1);
+    else if (a.K <= 6144 && !many) FG_W8_X(4, 6144, 8, 1);
+    else if (a.K <= 6144) FG_W8_X(4, 6144, 16, 1);
+    else if (a.K <= 7168) FG_W8_X(4, 7168, 8, 1);
+    else FG_W8_X(4, 8192, 16, 1);
+  } else if (a.M <= 8) {
+    if (a.K <= 512) FG_W8_X(8, 512, 4, 4);
+    else if (a.K <= 1024) FG_W8_X(8, 1024, 8, 3);
+    else if (a.K <= 1536) FG_W8_X(8, 1536, 4, 3);
+    else if (a.K <= 2048 && !many) FG_W8_X(8, 2048, 8, 1);
+    else if (a.K <= 2048) FG_W8_X(8, 2048, 4, 2);
+    else if (a.K <= 2560) FG_W8_X(8, 2560, 4, 2);
+    else if (a.K <= 3072) FG_W8_X(8, 3072, 8, 2);
+    else if (a.K <= 4096 && !many) FG_W8_X(8, 4096, 8, 1);
+    else if (a.K <= 4096) FG_W8_X(8, 4096, 16, 1);
+    else if (a.K <= 5120) FG_W8_X(8, 5120, 8, 1);
+    else if (a.K <= 6144) FG_W8_X(8, 6144, 8, 1);
+    else if (a.K <= 7168) FG_W8_X(8, 7168, 8, 1);
+    else FG_W8_X(8, 8192, 16, 1);
+  } else {
+    if (a.K <= 512) FG_W8_X(16, 512, 4, 4);
+    else if (a.K <= 1024) FG_W8_X(16, 1024, 4, 2);
+    else if (a.K <= 2048 && !many) FG_W8_X(16, 2048, 8, 1);
+    else if (a.K <= 2048) FG_W8_X(16, 2048, 4, 1);
+    else if (a.K <= 3072 && !many) FG_W8_X(16, 3072, 8, 1);
+    else if (a.K <= 3072) FG_W8_X(16, 3072, 4, 1);
+    else FG_W8_X(16, 4096, 16, 1);
+  }
+#undef FG_W8_X
+}
+
 // An earlier kernel with lanes along K (16 weight bytes a lane) against the row-load kernel on 256-byte
 // bands, us per call: K = N = 8192 M=1 12.6 / 14.3, M=2 15.1 / 14.2, M=4 21.1 / 14.9, M=8 32.9 / 17.2.
 // The row-load kernel exists with 8 waves only.
@@ -920,44 +1156,40 @@ bool launch_w8a16(const W8A16Args& a, hipStream_t s) {
   // 32-column tiles on 128-byte bands read half the activation bytes per weight byte.  Measured
   // against 16-column tiles (us):
   //  * two workgroups (16 waves) on every CU, 448..512 tiles or a multiple of 512: K = N = 16384 M=8
-  //    44.8 / 49.3, K=4096 N=16384 14.9 / 17.3, K=4096 N=14336 M=8 13.7 / 14.5 -- but not with rows
-  //    8 KB apart: K=8192 N=16384 M=8 27.6 / 25.2;
-  //  * one workgroup on every CU (N = 8192): long rows or 12..16 activation rows only (15..16 before three bands were in flight), K=16384 M=8
-  //    25.4 / 27.3, K=28672 M=14 47.8 / 55.4, K=4096 M=16 10.5 / 11.1, against K=8192 M=8 16.9 /
-  //    14.9, K=28672 M=4 40.0 / 38.7, K=2048 M=16 7.7 / 7.1;
+  //    44.8 / 49.3 -- but not with rows 8 KB apart: K=8192 N=16384 M=8 27.6 / 25.2;
+  //  * one workgroup on every CU (N = 8192): long rows or 12..16 activation rows only, K=16384 M=8
+  //    25.4 / 27.3, K=28672 M=14 47.8 / 55.4, against K=28672 M=4 40.0 / 38.7;
   //  * 13..16 rows from 160 tiles on: N=5120 K=11008 M=16 19.5 / 23.0, N=14336 K=14336 44.5 / 55.1.
   const bool aligned = a.N % 32 == 0;
   const bool two_per_cu = aligned && ((t32 >= 448 && t32 <= 512) || (t32 >= 512 && t32 % 512 == 0)) &&
                           (a.K != 8192 || a.M > 8);
   const bool one_per_cu = aligned && t32 == 256 &&
-                          ((a.M >= 12 && a.K >= 4096) || (a.K >= 16384 && (a.M >= 5 || a.K < 24576)));
+                          (a.M >= 12 || (a.K >= 16384 && (a.M >= 5 || a.K < 24576)));
   const bool many_rows = aligned && a.M >= 13 && t32 >= 160 && t32 != 256;
   const bool wide = two_per_cu || one_per_cu || many_rows;
   // 16-column tiles take 128-byte bands (smaller strips, more steps in flight): M=8, 128- / 256-byte
-  // bands: K = N = 8192 14.5 / 15.7, K = N = 4096 7.0 / 7.3, K=4096 N=14336 14.6 / 16.1, K=11008
-  // N=5120 17.7 / 19.3 -- except long rows of narrow outputs, K=14336 N=4096 M=4 14.8 / 13.9.
+  // bands: K=11008 N=5120 17.7 / 19.3 -- except long rows of narrow outputs, K=14336 N=4096 M=4 14.8 / 13.9.
   const bool bw256 = a.N <= 4096 && a.K >= 14336;
 #define FG_W8A16_R(XR, BW, CB)                                                                    \
   hipLaunchKernelGGL((w8a16_r_kernel<XR, 8, BW, CB>), dim3(a.N / (16 * CB)), dim3(512), 0, s, Wq, \
                      X, sc, a.scalar_scale, a.zero_point, Y, a.M, a.N, a.K)
   // Two rows run the lanes-over-x kernel on two rows -- except where the 16-column tiles of the row-load
-  // kernel fill the CUs evenly (us, two-row kernel / row-load kernel: N=4096 K=4096 6.0 / 7.1, K=14336
-  // 13.2 / 14.7; N=11008 K=4096 10.8 / 12.5; N=12288 K=3072 9.2 / 10.9, K=8192 20.0 / 20.8; N=28672 K=4096
-  // 22.0 / 24.0; N=2048 K=8192 6.1 / 6.8; N=1024 K=4096 3.7 / 4.5; but N=8192 K=8192 14.6 / 13.5, K=11008
-  // 18.4 / 17.0, K=4096 8.6 / 8.4, but K=2048 5.6 / 6.2; N=16384 K=8192 25.5 / 23.5; level at N=13824
-  // K=5120 and N=14336 K=4096).  Three and four rows only against narrow outputs, which leave the row-load kernel on
-  // half the CUs or fewer (M=4: N=1024 K=4096 4.5 / 5.3, N=2048 K=2048 4.3 / 5.6, K=8192 7.8 / 8.1;
-  // N=4096 K=4096 7.6 / 6.6 and N=8192 K=8192 23.2 / 13.7 the other way).
-  const bool even_tiles = a.N % 8192 == 0 && a.K >= 4096;
+  // kernel fill the CUs evenly (us, two-row kernel / row-load kernel: K=14336 N=4096 13.2 / 14.7; N=2048 K=8192
+  // 6.1 / 6.8; but N=8192 K=8192 14.6 / 13.5, K=11008 18.4 / 17.0; N=16384 K=8192 25.5 / 23.5).  Three and four
+  // rows only against narrow outputs, which leave the row-load kernel on half the CUs or fewer (M=4: N=1024
+  // K=4096 4.5 / 5.3, N=2048 K=8192 7.8 / 8.1).
+  const bool even_tiles = a.N % 8192 == 0;
   if (a.M == 1) {
     launch_wq_m1<8, 1>(a, s);
+  } else if (w8_panel(a)) {
+    launch_w8_panel(a, s);
   } else if (a.M == 2 && !even_tiles) {
     launch_wq_m1<8, 2>(a, s);
   } else if (a.M == 3 && a.N <= 2048) {
     launch_wq_m1<8, 3>(a, s);
   } else if (a.M == 4 && a.N <= 2048) {
     launch_wq_m1<8, 4>(a, s);
-  } else if (a.M <= 4) {  // 2 rows take the 4-row strip too: K=14336 N=4096 M=2 13.1 us
+  } else if (a.M <= 4) {  // (two rows take the 4-row strip too)
     if (wide) FG_W8A16_R(4, 128, 2);
     else if (bw256) FG_W8A16_R(4, 256, 1);
     else FG_W8A16_R(4, 128, 1);
@@ -968,11 +1200,10 @@ bool launch_w8a16(const W8A16Args& a, hipStream_t s) {
   } else if (a.M <= 16) {
     // 16-row activation strip on 128-byte bands only (the 256-byte form would need 100 KB of LDS).
     // 32-column tiles with three bands of a wave in flight instead of two (us): N = K = 8192 M=16 17.3 /
-    // 18.2, K=16384 25.9 / 27.5; N=16384 K=8192 31.3 / 32.7; N=14336 K=4096 17.2 / 18.1 -- with eight rows
-    // level or behind (N = K = 8192 15.3 / 14.7 against 16-column tiles, N=14336 K=4096 15.2 / 13.6), and
-    // 16-column tiles lose with any deeper pipeline (M=16 19.9 with three, 21.4 with four).  With three in
-    // flight the one-a-CU form at N = 8192 pays from 12 rows on (K=4096 M=12 9.8 / 10.6, K=8192 M=13 17.0 /
-    // 17.5; M=9 level).
+    // 18.2, K=16384 25.9 / 27.5; N=16384 K=8192 31.3 / 32.7 -- with eight rows level or behind (N = K = 8192
+    // 15.3 / 14.7 against 16-column tiles), and 16-column tiles lose with any deeper pipeline (M=16 19.9 with
+    // three, 21.4 with four).  With three in flight the one-a-CU form at N = 8192 pays from 12 rows on (K=8192
+    // M=13 17.0 / 17.5; M=9 level).
     if (wide)
       hipLaunchKernelGGL((w8a16_r_kernel<16, 8, 128, 2, 3>), dim3(a.N / 32), dim3(512), 0, s, Wq, X, sc,
                          a.scalar_scale, a.zero_point, Y, a.M, a.N, a.K);
@@ -1004,13 +1235,6 @@ static bool w4_panel(const W8A16Args& a) {
   if (a.K <= 8192) return a.M == 2 ? a.N > 2048 : a.N >= 1536;
   if (a.M == 2) return a.N >= 3072;
   return a.M == 4 ? a.N >= 1536 : (a.K <= 12288 ? a.N >= 2048 : a.N > 2048);
-}
-// Workgroups of a panel kernel: one a CU walks over up to `each` tiles, more where there are more tiles and LDS holds
-// them (`most`).  What a workgroup has in flight is one tile, 16 weight rows, and short rows leave a CU idle (int4 M=4
-// N=28672 K=2304 one / two a CU 11.9 / 8.9 us, K=1024 two / four 6.0 / 5.6), while for two tiles of longer rows a second
-// workgroup only stages the panel again (N=8192 K=3072 5.4 / 5.8, K=2048 3.9 / 4.2; K=1024 the other way, 3.4 / 3.3).
-static int panel_grid(int tiles, int cus, int each, int most) {
-  return std::min(tiles, cus * std::min(most, (tiles + each * cus - 1) / (each * cus)));
 }
 static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
   // KC: the smallest that holds K; four waves have enough to load up to K = 1024 (N=4096 3.1 / 2.7), sixteen share the
