@@ -293,11 +293,10 @@ __global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restric
                                                          int32_t* __restrict__ out, int M, int N, int K) {
   typedef int int4_v __attribute__((ext_vector_type(4)));
   constexpr int PAIRS = KC / 128 / NW;                // 16 rows x 128 bytes of weights: two loads a wave
-  // 1 KB of an activation row: one load a wave (fewer waves than rows: several rows a wave, one segment each)
-  constexpr bool kRows = NW < XR;
-  constexpr int SEGS = kRows ? XR / NW : (KC + 1023) / 1024 * XR / NW;
-  static_assert(KC % (128 * NW) == 0 && (KC % 1024 == 0 || KC < 1024) && (!kRows || KC <= 1024),
-                "whole pairs and segments");
+  // 1 KB of an activation row: one load a wave (fewer waves than rows: several rows a wave)
+  constexpr int ROWS = NW < XR ? XR / NW : 1;
+  constexpr int SEGS = ((KC + 1023) / 1024 * XR + NW - 1) / NW;
+  static_assert(KC % (128 * NW) == 0, "whole pairs");
   constexpr int STRIP = 2048, RED = XR * 16;          // ints a wave hands over
   constexpr bool kOwnRed = XR * KC + NW * (STRIP + 8 * RED) <= 160 * 1024;
   __shared__ u32x4 panel[XR * KC / 16];
@@ -311,14 +310,14 @@ __global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restric
   constexpr int kBeyond = 0x7ffffff0;                 // past the descriptors: the load returns zeros
   // activations first: loads return in order, and the panel must not wait for the weights
   // waves that stage a row: NW / M
-  int per_row = kRows ? 1 : NW / XR;
+  int per_row = NW < XR ? 1 : NW / XR;
   if constexpr (XR == 4) per_row = M == 2 ? NW / 2 : (M == 3 ? NW / 3 : NW / 4);
   else if constexpr (NW == 16) per_row = M == 5 ? 3 : 2;
-  const int xm = XR == 8 && NW <= 8 ? wave : wave / per_row, xs0 = kRows ? 0 : wave - xm * per_row;
+  const int xm = NW < XR ? wave * ROWS : wave / per_row, xs0 = wave - wave / per_row * per_row;
   u32x4 x[SEGS];
 #pragma unroll
   for (int i = 0; i < SEGS; ++i) {
-    const int row = xm + (kRows ? NW * i : 0), seg = xs0 + (kRows ? 0 : per_row * i);
+    const int row = xm + i % ROWS, seg = xs0 + per_row * (i / ROWS);
     const __amdgpu_buffer_rsrc_t xrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Xq + (size_t)row * K), 0, row < M ? K : 0, 0x00020000);
     x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, seg * 1024 + lane * 16, 0, 0));
@@ -348,7 +347,7 @@ __global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restric
   }
 #pragma unroll
   for (int i = 0; i < SEGS; ++i) {
-    const int row = xm + (kRows ? NW * i : 0), seg = xs0 + (kRows ? 0 : per_row * i);
+    const int row = xm + i % ROWS, seg = xs0 + per_row * (i / ROWS);
     const int q = seg * 64 + lane;                    // 16-k piece
     asm volatile("" : "+v"(x[i]));                    // (or the load sinks below the weights', to its only use)
     if (row < M && q < KC / 16) panel[q * XR + (row ^ ((q >> 2) & (XR - 1)))] = x[i];
@@ -1081,6 +1080,7 @@ static int panel_grid(int tiles, int cus, int each, int most) {
 //    N=11008 K=8192 18.0 / 16.4, N=3072 7.4 / 7.7;
 //  * not K > 6144 where 16-column tiles come out even, N = 8192 K=8192 four rows 12.9 / 13.2, two 11.5 / 11.9 at K=7168.
 static bool w8_panel(const W8A16Args& a) {
+
   const int tiles = a.N / 16, cus = compute_units(), rounds = (tiles + cus - 1) / cus;
   if (a.M >= 9) return a.K <= 4096;
   if (a.M >= 5) return a.K <= 6144 || (a.K <= 8192 && (8 * tiles <= 7 * cus || rounds > 1));
@@ -1096,7 +1096,7 @@ static void launch_w8_panel(const W8A16Args& a, hipStream_t s) {
   // KC: the smallest that holds K.  Few waves with several pairs each where that keeps loads enough in flight (us, eight
   // rows, one way / the other: N=8192 K=2560 eight waves of three pairs 6.7 / four of five 5.7; K=5120 sixteen waves 10.6
   // / eight of five 10.0; K=7168 12.4 sixteen / 11.5 eight of seven); more where one tile is all a workgroup does (N=1024
-  // K=2048 four / eight 3.7 / 3.5), and sixteen of two pairs at K = 4096 (N=8192 8.7 / 8.1 with eight of four).
+  // K=2048 four / eight 3.7 / 3.5), and at K = 4096 sixteen of two pairs (N=8192 eight of four 8.7 / 8.1).
   const int tiles = a.N / 16, cus = compute_units();
   const bool many = tiles > cus;
 #define FG_W8_X(XR, KC, NW, MOST)                                                                                  \
@@ -1118,6 +1118,7 @@ static void launch_w8_panel(const W8A16Args& a, hipStream_t s) {
     else if (a.K <= 6144) FG_W8_X(4, 6144, 16, 1);
     else if (a.K <= 7168) FG_W8_X(4, 7168, 8, 1);
     else FG_W8_X(4, 8192, 16, 1);
+
   } else if (a.M <= 8) {
     if (a.K <= 512) FG_W8_X(8, 512, 4, 4);
     else if (a.K <= 1024) FG_W8_X(8, 1024, 8, 3);
@@ -1237,20 +1238,29 @@ static bool w4_panel(const W8A16Args& a) {
   return a.M == 4 ? a.N >= 1536 : (a.K <= 12288 ? a.N >= 2048 : a.N > 2048);
 }
 static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
-  // KC: the smallest that holds K; four waves have enough to load up to K = 1024 (N=4096 3.1 / 2.7), sixteen share the
-  // largest panels (K=14336 10.8 / 10.4 with eight).
+  // KC: the smallest that holds K.  Few waves with several pairs each, the same number for every wave, where that keeps
+  // loads enough in flight (us, one way / the other): up to K = 1024 (N=4096 eight 3.1 / four 2.7), K=3072 N=4096 M=2
+  // eight of one or two 4.0 / four of three 3.5, K=5120 eight of two or three 5.0 / four of five 4.4 (but not beside it,
+  // K=4736 N=14336 8.8 / 9.9, nor with more tiles, N=20480 10.2 / 10.6), K=14336 N=8192 sixteen 15.2 / eight of seven
+  // 13.3, K=9216 sixteen 11.2 / eight of five 9.4.
   const int tiles = a.N / 16, cus = compute_units();
 #define FG_W4_X(KC, NW, MOST)                                                                                  \
   hipLaunchKernelGGL((w4a16_x_kernel<KC, NW>), dim3(panel_grid(tiles, cus, KC <= 1024 ? 1 : 2, MOST)), dim3(64 * NW), 0, s, \
                      static_cast<const uint8_t*>(a.Wq), static_cast<const half_t*>(a.x),                       \
                      static_cast<const half_t*>(a.scale), a.scalar_scale, a.zero_point, static_cast<half_t*>(a.y), \
                      a.M, a.N, a.K)
+  const bool many = tiles > cus;
   if (a.K <= 1024) FG_W4_X(1024, 4, 4);
   else if (a.K <= 2048) FG_W4_X(2048, 8, 2);
+  else if (a.K <= 3072) FG_W4_X(3072, 4, 2);
   else if (a.K <= 4096) FG_W4_X(4096, 8, 2);
+  else if (a.K > 4608 && a.K <= 5120 && tiles <= 2 * cus) FG_W4_X(5120, 4, 2);
   else if (a.K <= 6144) FG_W4_X(6144, 8, 1);
   else if (a.K <= 8192) FG_W4_X(8192, 8, 1);
-  else if (a.K <= 12288) FG_W4_X(12288, 16, 1);
+  else if (a.K <= 10240) FG_W4_X(10240, 8, 1);
+  else if (a.K <= 12288 && !many) FG_W4_X(12288, 16, 1);
+  else if (a.K <= 12288) FG_W4_X(12288, 8, 1);
+  else if (a.K <= 14336) FG_W4_X(14336, 8, 1);
   else FG_W4_X(16384, 16, 1);
 #undef FG_W4_X
 }
@@ -1324,17 +1334,24 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
 //    9.6 / 8.6; N=2048 K=14336 M=5 9.4 / 10.4, N=3072 M=8 14.4 / 11.7; N = K = 5120 11.4 / 7.3, N = K = 8192 15.9 / 12.4,
 //    N=14336 K=4096 16.6 / 11.3;
 //  * four: N=1024 K=4096 3.7 / 3.4, K=5120 4.0 / 4.4; N=1536 K=8192 5.7 / 5.6; N=2048 K=9216 6.9 / 7.3, N=3072 7.7 / 7.9; N =
-//    K = 5120 7.5 / 7.2, N=4096 K=8192 8.6 / 7.5, N=14336 K=4096 12.4 / 11.2, N = K = 8192 13.5 / 12.3; three, less: N=2048
-//    K=8192 6.0 / 5.8, N=9216 K=5120 10.0 / 10.3, N=5120 K=8192 9.4 / 9.6;
+//    K = 5120 7.5 / 7.2, N=4096 K=8192 8.6 / 7.5, N=14336 K=4096 12.4 / 11.2, N = K = 8192 13.5 / 12.3; three, less: N=2176
+//    K=7296 6.2 / 5.6, N=2048 K=7680 5.7 / 5.9, N=9216 K=5120 10.0 / 10.3, N=5120 K=8192 9.4 / 9.6 (the second round a quarter full).  To K =
+//    10240 where the rounds come out full: N=4096 three 9.8 / 9.0, four 10.2 / 9.1, N=8192 16.8 / 14.4; N=5120 11.3 / 12.0;
 //  * two, for which the v_dot4 kernel reads few activations: K <= 2048 (N=28672 10.9 / 10.3, N=2048 3.3 / 2.9), to K = 4096
 //    with one tile a CU at most (N=4096 5.2 / 4.7), to 6144 where one or two tiles a CU come out even (N=8192 9.6 / 9.0,
 //    N=7168 8.8 / 8.2; N=5120 7.3 / 7.7, N=9216 10.5 / 11.3).
 static bool i8_panel(int M, int N, int K) {
+
   if (M < 2 || K > 16384) return false;
   if (M >= 5) return K <= 4096 || N >= (K <= 6144 ? 1024 : (K <= 12288 ? 1536 : 2176));
   if (K <= 2048) return true;
-  if (M >= 3) return K <= 4096 ? N >= (M == 4 ? 512 : 1024) : (K <= 8192 && N >= (M == 4 ? 1536 : 2048));
   const int tiles = N / 16, cus = compute_units(), rounds = (tiles + cus - 1) / cus;
+  if (M >= 3) {
+    if (K <= 4096) return N >= (M == 4 ? 512 : 1024);
+    if (K <= 8192 && M == 4) return N >= 1536;
+    if (K <= 8192) return K <= 7168 ? N >= 2048 : (rounds == 1 ? N > 2048 : 8 * tiles > 5 * rounds * cus);
+    return K <= 10240 && 4 * tiles > 3 * rounds * cus;
+  }
   return (K <= 4096 && rounds == 1 && N >= 2048) || (K <= 6144 && rounds <= 2 && 8 * tiles >= 7 * rounds * cus);
 }
 
@@ -1344,7 +1361,9 @@ bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N,
   if (i8_panel(M, N, K)) {
     auto* W = static_cast<const int8_t*>(Wq);
     auto* X = static_cast<const int8_t*>(xq);
-    // Workgroups a CU as in launch_w4_panel.
+    // Workgroups a CU, and waves with the same number of pairs each, as in launch_w4_panel (eight rows, us, KC the next
+    // power of two or 6144, 12288 / as here: N=4096 K=2560 4.3 / 3.7, N=2048 K=3072 3.9 / 3.3, N = K = 5120 7.3 / 6.8,
+    // N=4096 K=7168 7.7 / 7.1, K=14336 13.3 / 12.7).
     const int tiles = N / 16, cus = compute_units();
 #define FG_I8_X(XR, KC, NW, MOST)                                                                    \
   hipLaunchKernelGGL((i8i8_x_kernel<XR, KC, NW>), dim3(panel_grid(tiles, cus, KC <= 1024 ? 1 : 2, MOST)), \
@@ -1352,17 +1371,30 @@ bool launch_i8i8_i32(const void* Wq, const void* xq, int32_t* acc, int M, int N,
     if (M <= 4) {
       if (K <= 512) FG_I8_X(4, 512, 4, 4);
       else if (K <= 1024) FG_I8_X(4, 1024, 4, 4);
+      else if (K <= 1536) FG_I8_X(4, 1536, 4, 4);
       else if (K <= 2048) FG_I8_X(4, 2048, 8, 3);
+      else if (K <= 2560) FG_I8_X(4, 2560, 4, 3);
+      else if (K <= 3072) FG_I8_X(4, 3072, 8, 2);
       else if (K <= 4096) FG_I8_X(4, 4096, 8, 2);
+      else if (K <= 5120) FG_I8_X(4, 5120, 8, 2);
       else if (K <= 6144) FG_I8_X(4, 6144, 8, 2);
-      else FG_I8_X(4, 8192, 8, 2);              // (longer rows: see i8_panel)
+      else if (K <= 7168) FG_I8_X(4, 7168, 8, 2);
+      else if (K <= 8192) FG_I8_X(4, 8192, 8, 2);
+      else FG_I8_X(4, 10240, 8, 1);             // (longer rows: see i8_panel)
     } else if (K <= 512) FG_I8_X(8, 512, 4, 4);
     else if (K <= 1024) FG_I8_X(8, 1024, 8, 3);
+    else if (K <= 1536) FG_I8_X(8, 1536, 4, 4);
     else if (K <= 2048) FG_I8_X(8, 2048, 8, 2);
+    else if (K <= 2560) FG_I8_X(8, 2560, 4, 3);
+    else if (K <= 3072) FG_I8_X(8, 3072, 8, 2);
     else if (K <= 4096) FG_I8_X(8, 4096, 8, 2);
+    else if (K <= 5120) FG_I8_X(8, 5120, 8, 1);
     else if (K <= 6144) FG_I8_X(8, 6144, 8, 1);
+    else if (K <= 7168) FG_I8_X(8, 7168, 8, 1);
     else if (K <= 8192) FG_I8_X(8, 8192, 8, 1);
+    else if (K <= 10240) FG_I8_X(8, 10240, 16, 1);
     else if (K <= 12288) FG_I8_X(8, 12288, 16, 1);
+    else if (K <= 14336) FG_I8_X(8, 14336, 16, 1);
     else FG_I8_X(8, 16384, 16, 1);
 #undef FG_I8_X
   } else if (M == 1) {

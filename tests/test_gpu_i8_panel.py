@@ -67,7 +67,10 @@ def test_lines_of_the_rule_are_exact(device, N, K):
                                  (8320, 2048), (8320, 2176), (12416, 4096), (4224, 4224), (8320, 5248), (8320, 8064),
                                  (512, 4096), (1024, 4096), (1024, 4224), (896, 6144), (1024, 6272), (1536, 8192),
                                  (1408, 8192), (1536, 8320), (2048, 12416), (2176, 12416), (3584, 5120), (3456, 5120),
-                                 (7168, 6144), (4224, 8192), (4224, 12288), (4224, 16384)])
+                                 (7168, 6144), (4224, 8192), (4224, 12288), (4224, 16384), (4224, 1152), (8320, 1536),
+                                 (2176, 2560), (8320, 2432), (4224, 3072), (4224, 5120), (2176, 5120), (2176, 7168),
+                                 (4224, 6272), (4096, 8320), (4096, 10240), (8192, 9344), (2176, 8320), (4224, 10240),
+                                 (4224, 14336), (4224, 12416)])
 def test_many_tiles_and_narrow_outputs_are_exact(device, N, K):
     g = torch.Generator(device=device)
     g.manual_seed(9850 + N + K)
