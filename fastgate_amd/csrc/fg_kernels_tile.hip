@@ -66,9 +66,16 @@ struct TileArgs {
   int ntiles, mblocks, splitk, xccs;
 };
 
+// PAIRED: several row blocks, which read the same weights side by side on one XCD.  In step they wait for the same
+// lines: each asks HBM for half of what its own CU could take.  So the odd ones walk K with the pairs of steps in each
+// four exchanged (2 3 0 1): either block brings half of the weights from HBM and finds the other half, two steps old,
+// in the L2.  For that the weights may not be non-temporal, and all tiles start at the same step: they read the same
+// activations at the same time.  us, M = 256, all in step / this: N=13824 K=5120 [K,N] 57.3 / 51.4, [N,K] 60.5 / 52.8;
+// N = K = 8192 [K,N] 63.1 / 54.0; M=200 4864 x 8320 49.9 / 36.8.  Loads alone 53 / 45.6; exchanging single steps or
+// fours, a start by XCD or by tile, or weights kept non-temporal (60.2) gave less.
 // FAR: [K,N] rows so far apart that the offsets over the rows of a step leave 32 bits (16 Mi elements and
 // more); the same steps and sums with 64-bit addresses for the weights.
-template <bool KN, bool FAR, int BM, int BN, int BK, int WM, int WN, int WK, int P>
+template <bool KN, bool FAR, bool PAIRED, int BM, int BN, int BK, int WM, int WN, int WK, int P>
 __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int TM = BM / WM, TN = BN / WN;  // wave tile
@@ -139,13 +146,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
 
   u32x4 ra[P][AI], rw[P][WI];
   // step numbers wrap around from a start that differs from tile to tile: rows are a power of two
-  // apart for the usual K, and workgroups in lockstep would sit on the same memory channels
-  int step = count > 0 ? tile % count : 0, issued = 0;
+  // apart for the usual K, and workgroups in lockstep would sit on the same memory channels (PAIRED: see above)
+  const int start = PAIRED || count == 0 ? 0 : tile % count;
+  const int swapped = PAIRED && (mblk & 1) ? count & ~3 : 0;
+  int issued = 0;
   auto load = [&](u32x4(&a)[AI], u32x4(&w)[WI]) {
-    constexpr int kNonTemporal = 2;  // the nt bit of a buffer load's cache policy
-    const bool live = issued++ < count;
+    constexpr int kNonTemporal = PAIRED ? 0 : 2;  // the nt bit of a buffer load's cache policy
+    const bool live = issued < count;
+    int step = start + (issued < swapped ? issued ^ 2 : issued);
+    if (step >= count) step -= count;
+    ++issued;
     const int k0 = (s0 + (FAR && !live ? 0 : step)) * BK;
-    step = step + 1 == count ? 0 : step + 1;
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t*>(Wt + (KN ? (size_t)k0 * t.ldw : (size_t)k0)), 0,
         (int)(live ? w_bytes - (KN ? 0u : (unsigned)k0 * 2u) : 0u), 0x00020000);
@@ -155,7 +166,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
     for (int i = 0; i < WI; ++i) {
       if constexpr (FAR) {  // (a step behind the last one reads the first again; it is never multiplied)
         const int c = i * NT + tid;
-        w[i] = load16<true>(Wt + (size_t)(k0 + c / WPR) * t.ldw + c % WPR * 8);
+        w[i] = load16<!PAIRED>(Wt + (size_t)(k0 + c / WPR) * t.ldw + c % WPR * 8);
       } else {
         w[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)w_off[i], 0, kNonTemporal));
       }
@@ -353,9 +364,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
 template <bool KN, bool FAR, int BM, int BN, int BK, int WM, int WN, int WK, int P>
 void tile_go(const TileArgs& t, hipStream_t s) {
   const int units = t.ntiles * t.splitk;
-  const unsigned grid = (unsigned)((units + t.xccs - 1) / t.xccs * t.xccs) * (unsigned)t.mblocks;
-  hipLaunchKernelGGL((tile_kernel<KN, FAR, BM, BN, BK, WM, WN, WK, P>), dim3(grid),
-                     dim3(64 * WM * WN * WK), 0, s, t);
+  const dim3 grid((unsigned)((units + t.xccs - 1) / t.xccs * t.xccs) * (unsigned)t.mblocks), block(64 * WM * WN * WK);
+  // Two row blocks over all of K gain nothing with the largest tile on short rows (K < 2048; M=200 N=14336 K=1024 14.4 /
+  // 14.9 us, while K=2048 N=28672 50.0 / 46.4), and lose where [N,K] rows 4 KB apart or a multiple of it put all tiles, in
+  // step, on the same channels (M=149 N=8192 K=2048 14.2 / 15.3, M=160 N = K = 8192 51.4 / 54.5; [K,N] 51.4 / 49.4).
+  const bool whole = t.mblocks == 2 && t.splitk == 1;
+  if (t.mblocks > 1 && !(whole && ((BM * BN >= 128 * 128 && t.K < 2048) || (!KN && t.K % 2048 == 0))))
+    hipLaunchKernelGGL((tile_kernel<KN, FAR, true, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
+  else
+    hipLaunchKernelGGL((tile_kernel<KN, FAR, false, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
 }
 
 }  // namespace

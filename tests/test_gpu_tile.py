@@ -255,3 +255,24 @@ def test_library_plans_of_the_tiled_kernel(device, layout, M, N, K, form):
         C = torch.full((M, N), float("nan"), dtype=torch.half, device=device)
         capi_gemm(A, W, C, layout, plan=p)
         assert torch.equal(C, _product(A, W, layout).half()), splitk
+
+
+# row blocks that share weight tiles walk K in exchanged steps (2 3 0 1): every remainder of the fours, K ranges of a
+# split that start anywhere, two and three blocks, both sides of the rule for two whole ones
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("form", FORMS)
+def test_row_blocks_side_by_side_are_exact(device, layout, form):
+    rows = (32, 32, 64, 96, 128, 128, 64)[form]
+    for N, K in ((384, 128), (384, 256), (640, 384), (384, 640), (640, 896), (384, 1920), (384, 2048), (384, 2304)):
+        for M in (rows + 1, 2 * rows, 2 * rows + 3):
+            A, W = _inputs(M, N, K, layout, device, whole=True)
+            exact = _product(A, W, layout).half()
+            for splitk in (1, 2, 5):
+                p = make_plan(capi.FG_KERNEL_KN_MFMA, tile_n=128, m_block=16, waves=8, splitk=splitk,
+                              stagger=2 + form) if layout == KN else \
+                    make_plan(capi.FG_KERNEL_NK_MFMA_R, tile_n=64, m_block=32, waves=8, splitk=splitk,
+                              stagger=2 + form, band=128)
+                C = torch.full((M + 1, N), -7.0, dtype=torch.half, device=device)
+                capi_gemm(A, W, C[:M], layout, plan=p)
+                assert torch.equal(C[:M], exact), (M, N, K, splitk)
+                assert bool((C[M] == -7.0).all())
