@@ -314,6 +314,7 @@ int fg_gemv_w8a16(const void* Wq, const void* x, const void* scale, float scalar
   if ((reinterpret_cast<uintptr_t>(Wq) | reinterpret_cast<uintptr_t>(x)) & 15) {
     return FG_ERR_INVALID_ARG;
   }
+  fg::read_compute_units();
   fg::W8A16Args a{Wq, x, scale, scalar_scale, zero_point, y, M, N, K};
   (void)hipGetLastError();
   if (!fg::launch_w8a16(a, static_cast<hipStream_t>(stream))) return FG_ERR_UNSUPPORTED;
