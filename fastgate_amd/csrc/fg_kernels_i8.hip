@@ -4,7 +4,8 @@
 //    subnormals (a byte or nibble in the low mantissa bits under a zero exponent is that number
 //    times 2^-24, exactly; see wq_m1_kernel), products and sums are fp32, and the per-output-channel
 //    scale and the zero point are applied once per output.
-//  * i8i8: int8 activations, v_dot4_i32_i8, exact int32 result.
+//  * i8i8: int8 activations, v_dot4_i32_i8 or the int8 MFMA, exact int32 result.
+//  * Two activation rows and more, where the activations fit LDS: the panel kernels (*_x_kernel).
 //
 // Replaces the device side of gemv_quantized_int8 (backend/cuda/hk/fastgemv.cuh:316-389,
 // 8-byte loads, int8 -> fp32 convert, scalar FMAs) of the reference.
@@ -286,14 +287,14 @@ __global__ __launch_bounds__(256) void i8i8_kernel(const int8_t* __restrict__ Wq
 // What bounds it: the weights at what memory gives (N = K = 8192 M=8 12.4 us, 5.4 TB/s, a plain read 11.9), on
 // short calls launch, one memory latency for the panel and one for the weights (N=4096 K=2048 3.3).  Measured against
 // a panel kernel with loads in operand order (18 instead of 64 bytes a clock a CU, see w4a16_x_kernel) and one tile a
-// workgroup, us: M=8 N = K = 8192 15.9 / 12.4, N=14336 K=4096 16.6 / 11.3, N = K = 5120 11.4 / 7.3, N=4096 K=2048 3.7 /
-// 3.3; M=4, the v_dot4 kernel, N = K = 8192 13.5 / 12.3, N=8192 K=4096 8.7 / 7.3, N = K = 5120 7.5 / 7.2.
+// workgroup, us: M=8 N = K = 8192 15.9 / 12.4, N=14336 K=4096 16.6 / 11.3, N = K = 5120 11.4 / 6.8, N=4096 K=2048 3.7 /
+// 3.3; M=4, the v_dot4 kernel, N = K = 8192 13.5 / 12.3, N=8192 K=4096 8.7 / 7.3, N = K = 5120 7.5 / 6.8.
 template <int XR, int KC, int NW>
 __global__ __launch_bounds__(64 * NW) void i8i8_x_kernel(const int8_t* __restrict__ Wq, const int8_t* __restrict__ Xq,
                                                          int32_t* __restrict__ out, int M, int N, int K) {
   typedef int int4_v __attribute__((ext_vector_type(4)));
   constexpr int PAIRS = KC / 128 / NW;                // 16 rows x 128 bytes of weights: two loads a wave
-  // 1 KB of an activation row: one load a wave (fewer waves than rows: several rows a wave)
+  // loads of 1 KB of an activation row a wave (fewer waves than rows: of several rows)
   constexpr int ROWS = NW < XR ? XR / NW : 1;
   constexpr int SEGS = ((KC + 1023) / 1024 * XR + NW - 1) / NW;
   static_assert(KC % (128 * NW) == 0, "whole pairs");
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(256) void dequant_i32_f16_kernel(const int32_t* __r
 // of one weight row per lane, converted to 8 fp16 there, against 16 bytes of one activation row.
 // The activations are fetched once per 16 weight rows instead of once per 4, the dot products run
 // on the matrix pipe, and the VALU only converts.  16-column tiles, 8 waves interleaving over K.
-// XROWS = activation rows staged: 4, 8 or 16.
+// XROWS = activation rows staged: 4, 8 or 16.  Serves rows too long for w8a16_x_kernel's panel.
 // ---------------------------------------------------------------------------------------
 template <int XROWS, int NW, int BW, int CB, int DEPTH = 2>
 __global__ __launch_bounds__(64 * NW) void w8a16_r_kernel(const int8_t* __restrict__ Wq,
@@ -1035,7 +1036,7 @@ static int i8_waves(int K) {
 // Two activation rows of int4 (MR = 2) against the row-load MFMA kernel: 8192 x 8192 11.4 -> 10.6,
 // 4096 x 4096 5.7 -> 5.0, 4096 x 14336 11.6 -> 10.7, 28672 x 4096 level; the second row costs 2 us at
 // 8192 x 8192 because its x traffic (64 MiB from L2) is twice the weights'; eight weight rows a
-// workgroup to halve it lose more in occupancy (11.9).  int8 keeps its row-load kernel for two rows.
+// workgroup to halve it lose more in occupancy (11.9).  (Now only where the panel kernel does not pay.)
 template <int BITS, int MR>
 static void launch_wq_m1(const W8A16Args& a, hipStream_t s) {
   auto* Wq = static_cast<const uint8_t*>(a.Wq);

@@ -20,15 +20,15 @@
 //    (column tile, K range) get ids that differ by the XCD count, so they read the same weights
 //    through the same L2 at about the same time.
 // What bounds it (128 x 128 tile, 2 x 4 waves of 64 x 32, 64 k a step, M = 256 N = 13824 K = 5120, counters
-// over the steps of one workgroup a CU): a step takes 1390 cycles.  The matrix cores are busy for 512
+// over the steps of one workgroup a CU, row blocks in step): a step takes 1390 cycles.  The matrix cores are busy for 512
 // of them, the LDS for 650 (every wave reads 64 + 32 rows, 96 KB in all, and 32 KB are written; no bank
 // conflicts), the loads take about 650 (32 KB at the 50 bytes a clock a CU takes from L2).  None of the
 // three is full: two waves a SIMD meet at a barrier every step, a wave spends a quarter of its time
 // ([N,K]: a sixth) waiting to issue to the LDS, and reads and products overlap only in part.
 // 64 x 64 wave tiles would read 64 KB.  K-splitting the waves (WK) halves the operand reads of the
 // narrow tiles, where every wave would otherwise read all rows.
-// Measured (us, the kernels for few rows repeated / this one): [K,N] M=256 N=13824 K=5120 333 / 58 (625
-// TFLOP/s; a large product through the vendor library reaches 1145 on the card), M=128 N = K = 8192
+// Measured (us, the kernels for few rows repeated / this one): [K,N] M=256 N=13824 K=5120 333 / 52..56 (645
+// TFLOP/s and more; a large product through the vendor library reaches 1145 on the card), M=128 N = K = 8192
 // 104 / 41; [N,K] M=48 N=4096 K=11008 40 / 21 (4.4 TB/s), M=96 N = K = 8192 91 / 34.
 // A split over K completes as for the other kernels: two passes, the counter protocol, or one
 // fixed-point atomic per element; partials are added in ascending order of the K range.
