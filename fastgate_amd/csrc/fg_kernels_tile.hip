@@ -70,13 +70,19 @@ struct TileArgs {
 // lines: each asks HBM for half of what its own CU could take.  So the odd ones walk K with the pairs of steps in each
 // four exchanged (2 3 0 1): either block brings half of the weights from HBM and finds the other half, two steps old,
 // in the L2.  For that the weights may not be non-temporal, and all tiles start at the same step: they read the same
-// activations at the same time.  us, M = 256, all in step / this: N=13824 K=5120 [K,N] 57.3 / 51.4, [N,K] 60.5 / 52.8;
-// N = K = 8192 [K,N] 63.1 / 54.0; M=200 4864 x 8320 49.9 / 36.8.  Loads alone 53 / 45.6; exchanging single steps or
-// fours, a start by XCD or by tile, or weights kept non-temporal (60.2) gave less.
+// activations at the same time.
+// A row's result must not depend on the block it lies in, so either order gives the same bits: steps 0 and 1 of each four
+// go into one sum, 2 and 3 into another, and the two meet once, after the last whole four (a + b is b + a); the steps
+// behind it go in order.  One sum in the order of the walk / two, us: [K,N] M=256 N=13824 K=5120 53.9 / 54.1, [N,K]
+// 54.9 / 53.1; 0.3 % more over 355 sizes of 33..512 rows (the worst M=419 N=2176 K=7040 39.9 / 42.6).
+// us, all in step / this, call after call: M=256 N=13824 K=5120 [K,N] 57.8 / 54.1, [N,K] 60.2 / 53.1; N = K = 8192 [K,N]
+// 64.5 / 57.9; M=200 N=4864 K=8320 [N,K] 49.2 / 38.4.  Loads alone 53 / 45.6; exchanging single steps or fours, a start
+// by XCD or by tile, or weights kept non-temporal (60.2) gave less.
 // FAR: [K,N] rows so far apart that the offsets over the rows of a step leave 32 bits (16 Mi elements and
 // more); the same steps and sums with 64-bit addresses for the weights.
 template <bool KN, bool FAR, bool PAIRED, int BM, int BN, int BK, int WM, int WN, int WK, int P>
-__global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
+__global__ __launch_bounds__(64 * WM * WN * WK, PAIRED && !FAR && BM == 64 && BN / WN == 32 ? 4 : 2)  // (two workgroups a CU)
+void tile_kernel(TileArgs t) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int TM = BM / WM, TN = BN / WN;  // wave tile
   constexpr int MB = TM / 16, NB = TN / 16;
@@ -185,11 +191,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
       *reinterpret_cast<u32x4*>(b + a_lds[i]) = a[i];
   };
 
-  float4_t acc[NB][MB];
+  constexpr int HALVES = PAIRED ? 2 : 1;     // (see PAIRED)
+  float4_t sums[HALVES][NB][MB];
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+  for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-    for (int m = 0; m < MB; ++m) acc[b][m] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) sums[h][b][m] = float4_t{0.f, 0.f, 0.f, 0.f};
+  float4_t(&acc)[NB][MB] = sums[0];
 
   const int a_rd = (wm * TM + j) * RS;
   const int w_rd = ABYTES + (wn * TN + j) * RS;  // [N,K]
@@ -219,18 +229,21 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
 #pragma unroll
     for (int m = 0; m < MB; ++m) av[set][m] = *reinterpret_cast<const u32x4*>(b + a_rd + m * 16 * RS + 16 * ((4 * u + g) ^ (j & SW)));
   };
-  auto multiply = [&](int set) {
+  auto multiply = [&](int set, int half = 0) {
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int m = 0; m < MB; ++m)
-        acc[i][m] =
-            __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wv[set][i]), as_half8(av[set][m]), acc[i][m], 0, 0, 0);
+        sums[half][i][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wv[set][i]), as_half8(av[set][m]),
+                                                                  sums[half][i][m], 0, 0, 0);
   };
+  auto clear_operands = [&](int set) {
 #pragma unroll
-  for (int i = 0; i < NB; ++i) wv[1][i] = u32x4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < NB; ++i) wv[set][i] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int m = 0; m < MB; ++m) av[1][m] = u32x4{0u, 0u, 0u, 0u};
+    for (int m = 0; m < MB; ++m) av[set][m] = u32x4{0u, 0u, 0u, 0u};
+  };
+  clear_operands(1);
 
 #pragma unroll
   for (int p = 0; p < P; ++p) {
@@ -240,18 +253,20 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   park(0, ra[0], rw[0]);
   load(ra[0], rw[0]);
   __builtin_amdgcn_sched_barrier(0);
-  constexpr int U = P % 2 ? 2 * P : P;  // register sets and LDS buffers both have constant numbers inside
+  // register sets, LDS buffers and (PAIRED) the sum a step adds to have constant numbers inside a round
+  constexpr int U = PAIRED ? 4 : (P % 2 ? 2 * P : P);
+  static_assert(U % P == 0 && U % 2 == 0, "whole turns of the register sets and of the LDS buffers");
   // Order within a step: a unit's operand reads go out first, then the products of the unit read before
   // it, with the LDS writes and the global loads dealt out between them -- issued in one piece they
   // hold every wave at the load unit while the matrix cores idle.
   constexpr int PIECE_OPS = AI + WI, MFMAS = MB * NB, GAP = UNITS * MFMAS / (2 * PIECE_OPS);
-  auto one_step = [&](int u) {
+  auto one_step = [&](int u, bool fours) {
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int uu = 0; uu < UNITS; ++uu) {
       fetch((u * UNITS + uu) & 1, u & 1, uu);
-      multiply((u * UNITS + uu + 1) & 1);
+      multiply((u * UNITS + uu + 1) & 1, fours ? ((uu == 0 ? u + 3 : u) >> 1) & 1 : 0);
     }
     park((u + 1) & 1, ra[(u + 1) % P], rw[(u + 1) % P]);
     load(ra[(u + 1) % P], rw[(u + 1) % P]);
@@ -273,15 +288,25 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void tile_kernel(TileArgs t) {
   int it = 0;
   for (; it + U <= count; it += U) {  // whole rounds only: a way out inside would blur the counts again
 #pragma unroll
-    for (int u = 0; u < U; ++u) one_step(u);
+    for (int u = 0; u < U; ++u) one_step(u, PAIRED);
+  }
+  if constexpr (PAIRED) {
+    multiply(1, 1);  // (the last unit of the fours)
+    clear_operands(1);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) acc[i][m] += sums[1][i][m];
   }
 #pragma unroll
   for (int u = 0; u < U - 1; ++u) {
     if (it + u >= count) break;
-    one_step(u);
+    one_step(u, false);
   }
-  if ((count * UNITS) & 1) multiply(0);
-  else multiply(1);
+  if (!PAIRED || (count & 3)) {  // (the last unit; PAIRED, whole fours: they are through)
+    if ((count * UNITS) & 1) multiply(0);
+    else multiply(1);
+  }
 
   // acc[i][m][r]: column wn TN + 16 i + 4 g + r of row wm TM + 16 m + j of the tile.  The K groups of
   // waves meet in LDS, the upper half of them handing over to the lower half until one is left; the
@@ -369,10 +394,22 @@ void tile_go(const TileArgs& t, hipStream_t s) {
   // 14.9 us, while K=2048 N=28672 50.0 / 46.4), and lose where [N,K] rows 4 KB apart or a multiple of it put all tiles, in
   // step, on the same channels (M=149 N=8192 K=2048 14.2 / 15.3, M=160 N = K = 8192 51.4 / 54.5; [K,N] 51.4 / 49.4).
   const bool whole = t.mblocks == 2 && t.splitk == 1;
-  if (t.mblocks > 1 && !(whole && ((BM * BN >= 128 * 128 && t.K < 2048) || (!KN && t.K % 2048 == 0))))
-    hipLaunchKernelGGL((tile_kernel<KN, FAR, true, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
-  else
+  if (t.mblocks == 1 || (whole && ((BM * BN >= 128 * 128 && t.K < 2048) || (!KN && t.K % 2048 == 0)))) {
     hipLaunchKernelGGL((tile_kernel<KN, FAR, false, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
+    return;
+  }
+  // 64 x 128 with two sums: 32 x 64 a wave take 168 registers, one workgroup a CU; 32 x 32 a wave on all of K leave room
+  // for two, but read a third more from LDS.  [K,N] one a CU at most: 1.02..1.04 of one sum's time against 0.98..1.01, more:
+  // 1.02 against 1.11..1.17; [N,K] 0.97..1.0 against 0.96..1.17.  (Eight XCDs of 32 CUs whatever the library counts: a plan
+  // adds in the same order everywhere.)
+  if constexpr (BM == 64 && BN == 128) {
+    if (!KN || (units + 7) / 8 * t.mblocks > 32) {
+      hipLaunchKernelGGL((tile_kernel<KN, FAR, true, BM, BN, BK, 2, 4, 1, P>), grid, block, 0, s, t);
+      return;
+    }
+  }
+  if constexpr (KN || BM != 64 || BN != 128)
+    hipLaunchKernelGGL((tile_kernel<KN, FAR, true, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
 }
 
 }  // namespace

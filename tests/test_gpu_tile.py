@@ -276,3 +276,34 @@ def test_row_blocks_side_by_side_are_exact(device, layout, form):
                 capi_gemm(A, W, C[:M], layout, plan=p)
                 assert torch.equal(C[:M], exact), (M, N, K, splitk)
                 assert bool((C[M] == -7.0).all())
+
+
+# a row's sums do not depend on the row block it lies in: equal rows give equal bits, whatever block of a call they are
+# in, and again in the next call.  Every remainder of the fours, K ranges of a split, few and many workgroups
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("form", FORMS)
+def test_equal_rows_give_equal_bits(device, layout, form):
+    rows = (32, 32, 64, 96, 128, 128, 64)[form]
+    M, distinct = 3 * rows + 5, 7
+    pick = torch.arange(M, device=device) % distinct
+    for N, K in ((640, 640), (640, 1152), (384, 1664), (640, 2304), (384, 4096), (8320, 1024)):
+        A, W = _inputs(distinct, N, K, layout, device, seed=form)
+        for splitk in (1, 3, 5):
+            p = make_plan(capi.FG_KERNEL_KN_MFMA, tile_n=128, m_block=16, waves=8, splitk=splitk, stagger=2 + form) if \
+                layout == KN else make_plan(capi.FG_KERNEL_NK_MFMA_R, tile_n=64, m_block=32, waves=8, splitk=splitk,
+                                            stagger=2 + form, band=128)
+            C = torch.empty((M, N), dtype=torch.half, device=device)
+            for _ in range(2):
+                capi_gemm(A[pick].contiguous(), W, C, layout, plan=p)
+                _close(C[:distinct], _product(A, W, layout), (N, K, splitk))
+                assert torch.equal(C, C[:distinct][pick]), (N, K, splitk)
+
+
+@pytest.mark.parametrize("layout", [KN, NK])
+@pytest.mark.parametrize("M,N,K", [(256, 13824, 1152), (256, 5120, 5120), (160, 10240, 1664), (48, 1024, 4736)])
+def test_equal_rows_of_the_librarys_plans_give_equal_bits(device, layout, M, N, K):
+    pick = torch.arange(M, device=device) % 7
+    A, W = _inputs(7, N, K, layout, device)
+    C = torch.empty((M, N), dtype=torch.half, device=device)
+    capi_gemm(A[pick].contiguous(), W, C, layout)
+    assert torch.equal(C, C[:7][pick])
