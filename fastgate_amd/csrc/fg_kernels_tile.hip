@@ -390,11 +390,25 @@ template <bool KN, bool FAR, int BM, int BN, int BK, int WM, int WN, int WK, int
 void tile_go(const TileArgs& t, hipStream_t s) {
   const int units = t.ntiles * t.splitk;
   const dim3 grid((unsigned)((units + t.xccs - 1) / t.xccs * t.xccs) * (unsigned)t.mblocks), block(64 * WM * WN * WK);
-  // Two row blocks over all of K gain nothing with the largest tile on short rows (K < 2048; M=200 N=14336 K=1024 14.4 /
-  // 14.9 us, while K=2048 N=28672 50.0 / 46.4), and lose where [N,K] rows 4 KB apart or a multiple of it put all tiles, in
-  // step, on the same channels (M=149 N=8192 K=2048 14.2 / 15.3, M=160 N = K = 8192 51.4 / 54.5; [K,N] 51.4 / 49.4).
-  const bool whole = t.mblocks == 2 && t.splitk == 1;
-  if (t.mblocks == 1 || (whole && ((BM * BN >= 128 * 128 && t.K < 2048) || (!KN && t.K % 2048 == 0)))) {
+  // Several row blocks exchange their steps (see PAIRED) but where that measured behind; 1900 calls of 33..4096 rows, their
+  // time exchanged / in step on average 0.93, us of the worst in step / exchanged:
+  //  * [K,N], 128 x 128 tiles of two to four blocks with K <= 2048, too few steps to pay: 1.02 (M=160 N=14336 K=1024 13.8 /
+  //    14.9); five blocks and more gain there too (M=2048 N=4096 K=2048 46.4 / 43.8).  [N,K], two blocks, K < 2048: level,
+  //    1.05..1.1 at worst (M=256 N=28672 K=512 19.7 / 21.7).
+  //  * [N,K] rows a power of two apart, from 4 KB on: all tiles start in step, on the same channels.  With two blocks of the
+  //    smaller tiles (three of 64 x 128) that costs as much as the exchange gives or more: up to 64 columns and rows 1.04
+  //    (M=64 N=8192 K=2048 10.2 / 12.2, K=16384 N=1024 in eight splits 12.9 / 14.1), 96 and 128 rows over all of K 0.81 at
+  //    K=4096 but 1.02..1.09 at K = 2048 and 8192 (M=160 N=8192 14.0 / 15.3, 44.2 / 46.7), split 0.98; 64 x 128 1.03
+  //    (M=149 N=10240 K=8192 50.2 / 53.9).  With more blocks the exchange wins there as well (K=2048 0.94, 4096 0.94,
+  //    8192 0.83; split 0.99, 0.95, 0.90; worst M=350 N=10240 K=2048 22.4 / 22.8), and with 128 x 128 tiles of two (0.94).
+  // The worst that is exchanged all the same: [K,N] M=400 N=4096 K=3072 19.7 / 21.0, [N,K] M=160 N=4096 K=16384 in two splits
+  // 44.6 / 49.4.
+  const bool largest = BM * BN >= 128 * 128, smallest = BM * BN <= 64 * 64;
+  const bool power_apart = !KN && t.K % 2048 == 0 && (t.K & (t.K - 1)) == 0;
+  const bool in_step = largest ? (KN ? t.K <= 2048 && t.mblocks <= 4 : t.K < 2048 && t.mblocks == 2)
+                               : power_apart && t.mblocks <= (BM == 64 && BN == 128 ? 3 : 2) &&
+                                     (t.splitk == 1 || smallest);
+  if (t.mblocks == 1 || in_step) {
     hipLaunchKernelGGL((tile_kernel<KN, FAR, false, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
     return;
   }

@@ -258,13 +258,13 @@ def test_library_plans_of_the_tiled_kernel(device, layout, M, N, K, form):
 
 
 # row blocks that share weight tiles walk K in exchanged steps (2 3 0 1): every remainder of the fours, K ranges of a
-# split that start anywhere, two and three blocks, both sides of the rule for two whole ones
+# split that start anywhere, two, three and five blocks, both sides of the rule between the two walks
 @pytest.mark.parametrize("layout", [KN, NK])
 @pytest.mark.parametrize("form", FORMS)
 def test_row_blocks_side_by_side_are_exact(device, layout, form):
     rows = (32, 32, 64, 96, 128, 128, 64)[form]
     for N, K in ((384, 128), (384, 256), (640, 384), (384, 640), (640, 896), (384, 1920), (384, 2048), (384, 2304)):
-        for M in (rows + 1, 2 * rows, 2 * rows + 3):
+        for M in (rows + 1, 2 * rows, 2 * rows + 3, 4 * rows + 3):
             A, W = _inputs(M, N, K, layout, device, whole=True)
             exact = _product(A, W, layout).half()
             for splitk in (1, 2, 5):
@@ -286,7 +286,7 @@ def test_equal_rows_give_equal_bits(device, layout, form):
     rows = (32, 32, 64, 96, 128, 128, 64)[form]
     M, distinct = 3 * rows + 5, 7
     pick = torch.arange(M, device=device) % distinct
-    for N, K in ((640, 640), (640, 1152), (384, 1664), (640, 2304), (384, 4096), (8320, 1024)):
+    for N, K in ((640, 640), (640, 1152), (384, 1664), (640, 2304), (384, 4096), (384, 6144), (8320, 1024)):
         A, W = _inputs(distinct, N, K, layout, device, seed=form)
         for splitk in (1, 3, 5):
             p = make_plan(capi.FG_KERNEL_KN_MFMA, tile_n=128, m_block=16, waves=8, splitk=splitk, stagger=2 + form) if \
