@@ -1336,14 +1336,16 @@ static void i8i8_go(const void* Wq, const void* xq, int32_t* acc, int M, int N, 
 //    9.6 / 8.6; N=2048 K=14336 M=5 9.4 / 10.4, N=3072 M=8 14.4 / 11.7; N = K = 5120 11.4 / 7.3, N = K = 8192 15.9 / 12.4,
 //    N=14336 K=4096 16.6 / 11.3;
 //  * four: N=1024 K=4096 3.7 / 3.4, K=5120 4.0 / 4.4; N=1536 K=8192 5.7 / 5.6; N=2048 K=9216 6.9 / 7.3, N=3072 7.7 / 7.9; N =
-//    K = 5120 7.5 / 7.2, N=4096 K=8192 8.6 / 7.5, N=14336 K=4096 12.4 / 11.2, N = K = 8192 13.5 / 12.3; three, less: N=2176
-//    K=7296 6.2 / 5.6, N=2048 K=7680 5.7 / 5.9, N=9216 K=5120 10.0 / 10.3, N=5120 K=8192 9.4 / 9.6 (the second round a quarter full).  To K =
-//    10240 where the rounds come out full: N=4096 three 9.8 / 9.0, four 10.2 / 9.1, N=8192 16.8 / 14.4; N=5120 11.3 / 12.0;
+//    K = 5120 7.5 / 7.2, N=4096 K=8192 8.6 / 7.5, N=14336 K=4096 12.4 / 11.2, N = K = 8192 13.5 / 12.3;
+//  * three, less: N=2176 K=7296 6.2 / 5.6, N=2048 K=7680 5.7 / 5.9, N=9216 K=5120 10.0 / 10.3; K > 7168 not where the second
+//    or third round is a quarter full or less (N=5120 K=8192 9.4 / 9.6, N=8320 K=7808 13.2 / 14.0, against N=5632 0.94 and
+//    N=9728 0.98 of the v_dot4 kernel's time);
+//  * three and four to K = 10240 where the rounds come out full: N=4096 three 9.8 / 9.0, four 10.2 / 9.1, N=8192 16.8 / 14.4;
+//    N=5120 11.3 / 12.0;
 //  * two, for which the v_dot4 kernel reads few activations: K <= 2048 (N=28672 10.9 / 10.3, N=2048 3.3 / 2.9), to K = 4096
 //    with one tile a CU at most (N=4096 5.2 / 4.7), to 6144 where one or two tiles a CU come out even (N=8192 9.6 / 9.0,
 //    N=7168 8.8 / 8.2; N=5120 7.3 / 7.7, N=9216 10.5 / 11.3).
 static bool i8_panel(int M, int N, int K) {
-
   if (M < 2 || K > 16384) return false;
   if (M >= 5) return K <= 4096 || N >= (K <= 6144 ? 1024 : (K <= 12288 ? 1536 : 2176));
   if (K <= 2048) return true;
@@ -1351,7 +1353,7 @@ static bool i8_panel(int M, int N, int K) {
   if (M >= 3) {
     if (K <= 4096) return N >= (M == 4 ? 512 : 1024);
     if (K <= 8192 && M == 4) return N >= 1536;
-    if (K <= 8192) return K <= 7168 ? N >= 2048 : (rounds == 1 ? N > 2048 : 8 * tiles > 5 * rounds * cus);
+    if (K <= 8192) return K <= 7168 ? N >= 2048 : (rounds == 1 ? N > 2048 : rounds > 3 || 4 * tiles > (4 * rounds - 3) * cus);
     return K <= 10240 && 4 * tiles > 3 * rounds * cus;
   }
   return (K <= 4096 && rounds == 1 && N >= 2048) || (K <= 6144 && rounds <= 2 && 8 * tiles >= 7 * rounds * cus);

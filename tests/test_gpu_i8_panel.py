@@ -44,7 +44,7 @@ def test_few_rows_beside_the_panel_are_exact(device, N, K):
 
 # both sides of every line between the panel, one piece a wave, and two pieces a wave
 @pytest.mark.parametrize("N,K", [(8192, 2048), (8320, 2048), (14336, 512), (14336, 640), (28672, 1536), (28672, 1664),
-                                 (16384, 2048), (16512, 2048), (3072, 4096), (2944, 4096), (3072, 4224), (4096, 6144),
+                                 (16384, 2048), (16512, 2048), (8320, 7808), (9216, 8064), (9344, 8064), (3072, 4096), (2944, 4096), (3072, 4224), (4096, 6144),
                                  (4096, 6272), (4224, 4096), (8192, 4096), (16384, 4096), (8192, 7296), (8064, 8192),
                                  (8192, 8192), (12288, 11264), (12288, 11392), (12160, 11392), (12288, 12288),
                                  (2176, 12288), (2176, 12416)])
