@@ -28,9 +28,12 @@ def test_panel_sizes_are_exact(device, N, K):
         assert bool((acc[M] == -3).all())
 
 
-@pytest.mark.parametrize("N,K", [(2176, 2304), (2176, 4992), (3072, 6144), (4224, 9088), (5120, 5120), (2176, 8192)])
+# on 256 CUs the v_dot4 kernel runs, on three or four waves: two rows everywhere but at K = 2304; three rows at N=5120
+# K=8192, N=8320 K=7808 and K > 8192; four at K > 8192.  The panel kernel has the rest
+@pytest.mark.parametrize("N,K", [(2176, 2304), (2176, 4992), (3072, 6144), (4224, 9088), (5120, 5120), (2176, 8192),
+                                 (5120, 8192), (8320, 7808), (5120, 9216), (2176, 10368), (3072, 11264)])
 def test_few_rows_beside_the_panel_are_exact(device, N, K):
-    # the v_dot4 kernel on three or four waves: K that gives every wave a piece, and K that does not
+    # K that gives every wave of the v_dot4 kernel a piece, and K that does not
     g = torch.Generator(device=device)
     g.manual_seed(9700 + N + K)
     W = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8, device=device)

@@ -1,5 +1,5 @@
 """int4 weights against two to four activation rows held in LDS as one panel: K at and beside the panel
-sizes (and beyond the largest, where the row-load kernel takes over), one and two column blocks a
+sizes (and beyond the largest, where the row-load kernel takes over), one and several column tiles a
 workgroup.  Single weights picked out come back exactly; sums are held to the oracle."""
 import numpy as np
 import pytest
@@ -28,7 +28,7 @@ def _run(Wd, x, scale, scalar_scale, zp, device):
 
 
 @pytest.mark.parametrize("K", KS)
-@pytest.mark.parametrize("N", [2176, 7168])  # 16 columns a workgroup; 32 (224 workgroups)
+@pytest.mark.parametrize("N", [2176, 7168])  # 136 tiles of 16 columns, one a workgroup; 448, more than CUs
 def test_panel_sizes(device, N, K):
     g = torch.Generator(device=device)
     g.manual_seed(9300 + N + K)
@@ -96,11 +96,12 @@ def test_smallest_and_largest_activations_are_exact(device, N, K, unit):
 
 
 # tiles of 16 columns that a workgroup walks over: the last round partly filled, one to four workgroups a CU, every
-# panel size (the largest shares its LDS between the waves' strips and their sums)
+# panel size (the largest shares its LDS between the waves' strips and their sums; 12288 with sixteen waves, where there
+# are no more tiles than CUs, and with eight)
 @pytest.mark.parametrize("N,K", [(33024, 128), (17408, 1024), (33024, 896), (8320, 1152), (12416, 2048), (8320, 2176),
                                  (8320, 4224), (8320, 8192), (4224, 12160), (8320, 12416), (4224, 16384), (4224, 2176),
                                  (2176, 3072), (2176, 4736), (4224, 5120), (8320, 4992), (2176, 8320), (4224, 10240),
-                                 (2176, 12416), (4224, 14336)])
+                                 (2176, 12416), (4224, 14336), (4096, 11008), (3072, 12288), (24704, 1152)])
 def test_many_tiles_a_workgroup_are_exact(device, N, K):
     # |x| <= 8 and weights below 16: every sum is a whole number below 2^24, the scale a power of two
     g = torch.Generator(device=device)
