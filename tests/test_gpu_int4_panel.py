@@ -101,7 +101,8 @@ def test_smallest_and_largest_activations_are_exact(device, N, K, unit):
 @pytest.mark.parametrize("N,K", [(33024, 128), (17408, 1024), (33024, 896), (8320, 1152), (12416, 2048), (8320, 2176),
                                  (8320, 4224), (8320, 8192), (4224, 12160), (8320, 12416), (4224, 16384), (4224, 2176),
                                  (2176, 3072), (2176, 4736), (4224, 5120), (8320, 4992), (2176, 8320), (4224, 10240),
-                                 (2176, 12416), (4224, 14336), (4096, 11008), (3072, 12288), (24704, 1152)])
+                                 (2176, 12416), (4224, 14336), (4096, 11008), (3072, 12288), (24704, 1152), (2176, 4352),
+                                 (8320, 4352)])
 def test_many_tiles_a_workgroup_are_exact(device, N, K):
     # |x| <= 8 and weights below 16: every sum is a whole number below 2^24, the scale a power of two
     g = torch.Generator(device=device)
