@@ -1243,10 +1243,10 @@ static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
   // loads enough in flight (us, one way / the other): up to K = 1024 (N=4096 eight 3.1 / four 2.7), K=3072 N=4096 M=2
   // eight of one or two 4.0 / four of three 3.5, K=14336 N=8192 sixteen 15.2 / eight of seven 13.3, K=9216 sixteen 11.2 /
   // eight of five 9.4.  K = 4224..5120: eight waves of three pairs, or four of five where rows are whole lines (K a multiple
-  // of 256; the same loads touch fewer of them) and no CU has more than two tiles: 0.89..1.01 of the time of eight (N=4096
-  // K=5120 0.89, K=4352 0.91), with rows that end half way into a line 0.98..1.05, with more tiles 1.01..1.13.  K =
-  // 1152..2048: up to three workgroups a CU (240 calls 0.99 of the time with two; M=2 N=32768 K=1152 7.5 / 6.7, with one tile
-  // a workgroup 6.6); four waves instead, 1.02.
+  // of 256; the same loads touch fewer of them) and no CU has more than two tiles: 0.88..1.03 of the time of eight (N=4096
+  // K=5120 0.89, K=4352 0.91).  Rows that end half way into a line: three and four rows 0.98..1.08, two 0.95..1.01 from K =
+  // 4736 on; more tiles 1.01..1.13.  K = 1152..2048: up to three workgroups a CU (240 calls 0.99 of the time with two; M=2
+  // N=32768 K=1152 7.5 / 6.7, with one tile a workgroup 6.6); four waves instead, 1.02.
   const int tiles = a.N / 16, cus = compute_units();
 #define FG_W4_X(KC, NW, MOST)                                                                                  \
   hipLaunchKernelGGL((w4a16_x_kernel<KC, NW>), dim3(panel_grid(tiles, cus, KC <= 1024 ? 1 : 2, MOST)), dim3(64 * NW), 0, s, \
@@ -1258,7 +1258,7 @@ static void launch_w4_panel(const W8A16Args& a, hipStream_t s) {
   else if (a.K <= 2048) FG_W4_X(2048, 8, 3);
   else if (a.K <= 3072) FG_W4_X(3072, 4, 2);
   else if (a.K <= 4096) FG_W4_X(4096, 8, 2);
-  else if (a.K <= 5120 && a.K % 256 == 0 && tiles <= 2 * cus) FG_W4_X(5120, 4, 2);
+  else if (a.K <= 5120 && (a.K % 256 == 0 || (a.M == 2 && a.K > 4608)) && tiles <= 2 * cus) FG_W4_X(5120, 4, 2);
   else if (a.K <= 6144) FG_W4_X(6144, 8, 1);
   else if (a.K <= 8192) FG_W4_X(8192, 8, 1);
   else if (a.K <= 10240) FG_W4_X(10240, 8, 1);
