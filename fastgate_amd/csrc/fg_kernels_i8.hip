@@ -421,7 +421,8 @@ __global__ __launch_bounds__(256) void dequant_i32_f16_kernel(const int32_t* __r
 // of one weight row per lane, converted to 8 fp16 there, against 16 bytes of one activation row.
 // The activations are fetched once per 16 weight rows instead of once per 4, the dot products run
 // on the matrix pipe, and the VALU only converts.  16-column tiles, 8 waves interleaving over K.
-// XROWS = activation rows staged: 4, 8 or 16.  Serves rows too long for w8a16_x_kernel's panel.
+// XROWS = activation rows staged: 4, 8 or 16.  Serves what w8_panel leaves: rows too long for w8a16_x_kernel's panel, and
+// long ones whose tiles come out even on the CUs without one.
 // ---------------------------------------------------------------------------------------
 template <int XROWS, int NW, int BW, int CB, int DEPTH = 2>
 __global__ __launch_bounds__(64 * NW) void w8a16_r_kernel(const int8_t* __restrict__ Wq,
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(64 * NW) void w8a16_r_kernel(const int8_t* __restri
 // parked already paired the way the nibble conversion produces its halves -- (x0,x4),(x1,x5),
 // (x2,x6),(x3,x7) per 8 k -- so the 4 bytes a lane reads per MFMA unit turn into the B operand with
 // one shift, four v_and_or and four exact fp16 subtractions, and the dot products run on the
-// matrix pipe.  XROWS = activation rows staged (2 or 4).
+// matrix pipe.  XROWS = activation rows staged (4).
 // ---------------------------------------------------------------------------------------
 template <int XROWS>
 __global__ __launch_bounds__(512) void w4a16_r_kernel(const uint8_t* __restrict__ Wq,
@@ -705,10 +706,12 @@ __global__ __launch_bounds__(512) void w4a16_r_kernel(const uint8_t* __restrict_
 //  * The row sums for the zero point are taken while the panel is staged.
 // Loads return in order, so their order counts: activations, then the scales (cold), then the weights (the scales
 // last: 0.35 us more on every call).
-// What bounds it: N=4096 K=14336 M=4 9.9 us of which a call without any load or product takes 4.3, the weights
-// 3.4 more (29 MB), activations 1.2 (115 KB a CU from L2), decode and products after the last load 1.0.  Measured
-// against the same panel with the loads in operand order and one tile a workgroup (us): N=4096 K=14336 M=4
-// 11.8 / 9.9, N = K = 8192 10.9 / 8.8, N=14336 K=4096 9.1 / 7.9, N=28672 K=2304 11.2 / 8.9, N=4096 K=4096 4.4 / 4.1.
+// What bounds it: the way of the weights through LDS, one pair after the other in every wave (park, wait, read, decode,
+// multiply), which the loads hide only in part.  M=4, weights from memory, us: N=4096 K=14336 (eight waves, seven pairs each)
+// 9.6; an empty kernel of its LDS and waves 1.7, the kernel with every load answered by zeros at once 6.9, with the
+// activations' loads alone 7.1, with the weights' alone 9.0.  N = K = 8192 8.8, 1.7, 6.3, 6.2, 8.5; N = K = 4096 4.1, 1.7,
+// 3.6, 3.6, 3.9.  Against the same panel with the loads in operand order and one tile a workgroup: N=4096 K=14336 11.8 / 9.6,
+// N = K = 8192 10.9 / 8.8, N=14336 K=4096 9.1 / 7.9, N=28672 K=2304 11.2 / 8.9, N=4096 K=4096 4.4 / 4.1.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
   v = row16_allreduce(v);
@@ -746,7 +749,8 @@ __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restr
   u32x4 x[SEGS];
 #pragma unroll
   for (int i = 0; i < SEGS; ++i)
-    x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (xs0 + per_row * i) * 1024 + lane * 16, 0, 0));
+    x[i] = __builtin_bit_cast(
+        u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (xs0 + per_row * i) * 1024 + lane * 16, 0, 0));
   __builtin_amdgcn_sched_barrier(0);
 
   u32x4 w[PAIRS][2];
@@ -762,8 +766,9 @@ __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restr
         const_cast<uint8_t*>(Wq + (size_t)tile * 16 * rowb), 0, tile < tiles ? (int)(16 * rowb) : 0, 0x00020000);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      w[t][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                              wrs, w_off[t] == kBeyond ? kBeyond : w_off[t] + 8 * h * (int)rowb, 0, kNonTemporal));
+      w[t][h] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     wrs, w_off[t] == kBeyond ? kBeyond : w_off[t] + 8 * h * (int)rowb, 0, kNonTemporal));
   };
   int tile = blockIdx.x;
   // scale of the output this thread writes, ahead of the tile's weights
@@ -786,7 +791,8 @@ __global__ __launch_bounds__(64 * NW) void w4a16_x_kernel(const uint8_t* __restr
       for (int c = 0; c < 4; ++c) xsum = __builtin_amdgcn_fdot2(as_half2(a[c]), ones, xsum, false);
       constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;
       const int q = seg * 32 + (lane >> 1);      // 16-k group
-      u32x2* at = reinterpret_cast<u32x2*>(panel + (q >> 3) * 64 + (q & 1) * 32 + ((q >> 1) & 3) * 4 + (xm ^ ((q >> 3) & 3))) + (lane & 1);
+      const int piece = (q >> 3) * 64 + (q & 1) * 32 + ((q >> 1) & 3) * 4 + (xm ^ ((q >> 3) & 3));
+      u32x2* at = reinterpret_cast<u32x2*>(panel + piece) + (lane & 1);
       at[0] = u32x2{__builtin_amdgcn_perm(a.z, a.x, kLow), __builtin_amdgcn_perm(a.w, a.y, kLow)};
       at[32] = u32x2{__builtin_amdgcn_perm(a.z, a.x, kHigh), __builtin_amdgcn_perm(a.w, a.y, kHigh)};
     }
@@ -1081,7 +1087,6 @@ static int panel_grid(int tiles, int cus, int each, int most) {
 //    N=11008 K=8192 18.0 / 16.4, N=3072 7.4 / 7.7;
 //  * not K > 6144 where 16-column tiles come out even, N = 8192 K=8192 four rows 12.9 / 13.2, two 11.5 / 11.9 at K=7168.
 static bool w8_panel(const W8A16Args& a) {
-
   const int tiles = a.N / 16, cus = compute_units(), rounds = (tiles + cus - 1) / cus;
   if (a.M >= 9) return a.K <= 4096;
   if (a.M >= 5) return a.K <= 6144 || (a.K <= 8192 && (8 * tiles <= 7 * cus || rounds > 1));
@@ -1119,7 +1124,6 @@ static void launch_w8_panel(const W8A16Args& a, hipStream_t s) {
     else if (a.K <= 6144) FG_W8_X(4, 6144, 16, 1);
     else if (a.K <= 7168) FG_W8_X(4, 7168, 8, 1);
     else FG_W8_X(4, 8192, 16, 1);
-
   } else if (a.M <= 8) {
     if (a.K <= 512) FG_W8_X(8, 512, 4, 4);
     else if (a.K <= 1024) FG_W8_X(8, 1024, 8, 3);
@@ -1228,7 +1232,7 @@ bool launch_w8a16(const W8A16Args& a, hipStream_t s) {
 //    5.9 / 5.6;
 //  * K = 12288 N=1024 4.9 / 6.5, 5.8 / 6.8, 6.6 / 7.1, N=1536 6.2 / 6.7, 7.4 / 6.9, 10.7 / 7.2, N=3072 7.6 / 7.2;
 //  * K = 16384 N=1536 6.6 / 7.9, 7.8 / 8.4, 10.9 / 8.7, N=2048 6.9 / 8.1, 8.2 / 8.5, N=3072 8.9 / 8.7, 10.9 / 9.1.
-// Against the row-load kernel N=4096 K=14336 M=4 13.0, N = K = 8192 12.7, N=5120 K=11008 16.9 (this one 9.9, 8.8, 10.4).
+// Against the row-load kernel N=4096 K=14336 M=4 13.0, N = K = 8192 12.7, N=5120 K=11008 16.9 (this one 9.6, 8.8, 10.4).
 static bool w4_panel(const W8A16Args& a) {
   if (a.K > 16384) return false;
   if (a.K <= 2048) return true;
@@ -1283,8 +1287,7 @@ bool launch_w4a16(const W8A16Args& a, hipStream_t s) {
     launch_wq_m1<4, 2>(a, s);
   } else if (a.N <= 2048) {
     // narrow outputs leave the 16-column tiles of the row-load kernel on half the CUs or fewer (M=4, us,
-    // lanes-over-x / row-load: N=1024 K=4096 4.6 / 5.3, K=8192 5.3 / 7.4; N=2048 K=2048 4.3 / 5.0, K=8192
-    // 7.5 / 7.7; N=3072 K=3072 5.7 / 5.3 and N=4096 K=4096 6.6 / 5.7 the other way)
+    // lanes-over-x / row-load: N=1024 K=8192 5.3 / 7.4; towards 2048 columns they meet)
     if (a.M == 3) launch_wq_m1<4, 3>(a, s);
     else launch_wq_m1<4, 4>(a, s);
   } else {

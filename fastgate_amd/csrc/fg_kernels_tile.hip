@@ -6,9 +6,9 @@
 // 128), so the weights leave memory once, and its waves share both operands through LDS.
 //
 //  * Per step the workgroup stages BK k of its BN weight columns and of its BM activation rows:
-//    16-byte loads into registers, P steps ahead (weights non-temporal, activations from L2), from
-//    there into one of two LDS buffers -- one barrier a step.  Rows beyond M load as zeros
-//    and are never stored.
+//    16-byte loads into registers, P steps ahead (weights non-temporal unless row blocks exchange
+//    steps, activations from L2), from there into one of two LDS buffers -- one barrier a step.  Rows
+//    beyond M load as zeros and are never stored.
 //  * k-contiguous rows lie in LDS as 16-byte pieces permuted by their row, so the operand-order reads
 //    (ds_read_b128, row j, piece g) hit distinct banks without padding.  [K,N] rows lie as they come, 16 columns = 32 bytes a
 //    group, groups permuted by k so that the four k rows a transposing read (ds_read_b64_tr_b16)
@@ -18,7 +18,7 @@
 //    columns of one row of C (8-byte stores, 16-byte partials).
 //  * One-dimensional grid.  Workgroups go to the XCDs round-robin by id; the row blocks of one
 //    (column tile, K range) get ids that differ by the XCD count, so they read the same weights
-//    through the same L2 at about the same time.
+//    through the same L2 at about the same time (in exchanged steps, see PAIRED).
 // What bounds it (128 x 128 tile, 2 x 4 waves of 64 x 32, 64 k a step, M = 256 N = 13824 K = 5120, counters
 // over the steps of one workgroup a CU, row blocks in step): a step takes 1390 cycles.  The matrix cores are busy for 512
 // of them, the LDS for 650 (every wave reads 64 + 32 rows, 96 KB in all, and 32 KB are written; no bank
@@ -27,8 +27,8 @@
 // ([N,K]: a sixth) waiting to issue to the LDS, and reads and products overlap only in part.
 // 64 x 64 wave tiles would read 64 KB.  K-splitting the waves (WK) halves the operand reads of the
 // narrow tiles, where every wave would otherwise read all rows.
-// Measured (us, the kernels for few rows repeated / this one): [K,N] M=256 N=13824 K=5120 333 / 52..56 (645
-// TFLOP/s and more; a large product through the vendor library reaches 1145 on the card), M=128 N = K = 8192
+// Measured (us, the kernels for few rows repeated / this one): [K,N] M=256 N=13824 K=5120 333 / 54 (670
+// TFLOP/s; a large product through the vendor library reaches 1145 on the card), M=128 N = K = 8192
 // 104 / 41; [N,K] M=48 N=4096 K=11008 40 / 21 (4.4 TB/s), M=96 N = K = 8192 91 / 34.
 // A split over K completes as for the other kernels: two passes, the counter protocol, or one
 // fixed-point atomic per element; partials are added in ascending order of the K range.
@@ -81,7 +81,7 @@ struct TileArgs {
 // FAR: [K,N] rows so far apart that the offsets over the rows of a step leave 32 bits (16 Mi elements and
 // more); the same steps and sums with 64-bit addresses for the weights.
 template <bool KN, bool FAR, bool PAIRED, int BM, int BN, int BK, int WM, int WN, int WK, int P>
-__global__ __launch_bounds__(64 * WM * WN * WK, PAIRED && !FAR && BM == 64 && BN / WN == 32 ? 4 : 2)  // (two workgroups a CU)
+__global__ __launch_bounds__(64 * WM * WN * WK, PAIRED && !FAR && BM == 64 && BN / WN == 32 ? 4 : 2)  // (4: two a CU)
 void tile_kernel(TileArgs t) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int TM = BM / WM, TN = BN / WN;  // wave tile

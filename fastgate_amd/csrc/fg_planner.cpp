@@ -110,8 +110,10 @@ int pick_splitk(int tiles, int waves, int items, int M, int N, int K, int target
 // of bk k each; a split adds s0 + s2 S + s1 S M N / 2^20 (partials written and read again).  t1 is
 // what a step takes when a CU has one workgroup (latency), t2 what each takes when several keep it
 // busy.  Fitted, one form and layout at a time, to 4000 timings over sixteen (N, K) from 1024 x 4096 to
-// 28672 x 2048, twelve M from 17 to 256 and splits of 1 .. 16 (8 % rms); the form and split it picks
-// are on average 2 % slower than the best of that sweep.
+// 28672 x 2048, twelve M from 17 to 256 and splits of 1 .. 16 (8 % rms).  The timings are from before row blocks
+// exchanged their steps: calls of several blocks have become faster since, and the model does not know it.  What it picks
+// against the best form and split, 469 calls now: one row block 2.2 % slower on average, several 2.6 % ([K,N] 3.5, [N,K]
+// 1.5); the worst [K,N] M=256 N = K = 2048, 10.8 us against 8.2 (32 x 64 unsplit).
 struct TileCost {
   float c, c2, t1, t2, s0, s1, s2;
 };
