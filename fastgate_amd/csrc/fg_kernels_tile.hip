@@ -74,7 +74,7 @@ struct TileArgs {
 // A row's result must not depend on the block it lies in, so either order gives the same bits: steps 0 and 1 of each four
 // go into one sum, 2 and 3 into another, and the two meet once, after the last whole four (a + b is b + a); the steps
 // behind it go in order.  One sum in the order of the walk / two, us: [K,N] M=256 N=13824 K=5120 53.9 / 54.1, [N,K]
-// 54.9 / 53.1; 0.3 % more over 355 sizes of 33..512 rows (the worst M=419 N=2176 K=7040 39.9 / 42.6).
+// 54.9 / 53.1; level over 355 sizes of 33..512 rows (the worst M=419 N=2176 K=7040 39.8 / 41.8).
 // us, all in step / this, call after call: M=256 N=13824 K=5120 [K,N] 57.8 / 54.1, [N,K] 60.2 / 53.1; N = K = 8192 [K,N]
 // 64.5 / 57.9; M=200 N=4864 K=8320 [N,K] 49.2 / 38.4.  Loads alone 53 / 45.6; exchanging single steps or fours, a start
 // by XCD or by tile, or weights kept non-temporal (60.2) gave less.
@@ -160,7 +160,7 @@ void tile_kernel(TileArgs t) {
     constexpr int kNonTemporal = PAIRED ? 0 : 2;  // the nt bit of a buffer load's cache policy
     const bool live = issued < count;
     int step = start + (issued < swapped ? issued ^ 2 : issued);
-    if (step >= count) step -= count;
+    if (!PAIRED && step >= count) step -= count;
     ++issued;
     const int k0 = (s0 + (FAR && !live ? 0 : step)) * BK;
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
@@ -396,18 +396,19 @@ void tile_go(const TileArgs& t, hipStream_t s) {
   //    14.9); five blocks and more gain there too (M=2048 N=4096 K=2048 46.4 / 43.8).  [N,K], two blocks, K < 2048: level,
   //    1.05..1.1 at worst (M=256 N=28672 K=512 19.7 / 21.7).
   //  * [N,K] rows a power of two apart, from 4 KB on: all tiles start in step, on the same channels.  With two blocks of the
-  //    smaller tiles (three of 64 x 128) that costs as much as the exchange gives or more: up to 64 columns and rows 1.04
-  //    (M=64 N=8192 K=2048 10.2 / 12.2, K=16384 N=1024 in eight splits 12.9 / 14.1), 96 and 128 rows over all of K 0.81 at
-  //    K=4096 but 1.02..1.09 at K = 2048 and 8192 (M=160 N=8192 14.0 / 15.3, 44.2 / 46.7), split 0.98; 64 x 128 1.03
-  //    (M=149 N=10240 K=8192 50.2 / 53.9).  With more blocks the exchange wins there as well (K=2048 0.94, 4096 0.94,
-  //    8192 0.83; split 0.99, 0.95, 0.90; worst M=350 N=10240 K=2048 22.4 / 22.8), and with 128 x 128 tiles of two (0.94).
+  //    smaller tiles (three of 64 x 128) that costs as much as the exchange gives or more: up to 64 columns and rows 1.11
+  //    unsplit (M=64 N=8192 K=2048 10.2 / 12.2) and 1.02 split from K=8192 on (K=16384 N=1024 in eight 12.9 / 14.1; K=4096
+  //    0.97); 96 and 128 rows over all of K 0.81 at K=4096 but 1.02..1.09 at K = 2048 and 8192 (M=160 N=8192 14.0 / 15.3,
+  //    44.2 / 46.7), split 0.98; 64 x 128 1.03 (M=149 N=10240 K=8192 50.2 / 53.9).  With more blocks the exchange wins there
+  //    as well (K=2048 0.94, 4096 0.94, 8192 0.83; split 0.99, 0.95, 0.90; worst M=350 N=10240 K=2048 22.4 / 22.8), and with
+  //    128 x 128 tiles of two (0.94).
   // The worst that is exchanged all the same: [K,N] M=400 N=4096 K=3072 19.7 / 21.0, [N,K] M=160 N=4096 K=16384 in two splits
   // 44.6 / 49.4.
   const bool largest = BM * BN >= 128 * 128, smallest = BM * BN <= 64 * 64;
   const bool power_apart = !KN && t.K % 2048 == 0 && (t.K & (t.K - 1)) == 0;
   const bool in_step = largest ? (KN ? t.K <= 2048 && t.mblocks <= 4 : t.K < 2048 && t.mblocks == 2)
                                : power_apart && t.mblocks <= (BM == 64 && BN == 128 ? 3 : 2) &&
-                                     (t.splitk == 1 || smallest);
+                                     (t.splitk == 1 || (smallest && t.K >= 8192));
   if (t.mblocks == 1 || in_step) {
     hipLaunchKernelGGL((tile_kernel<KN, FAR, false, BM, BN, BK, WM, WN, WK, P>), grid, block, 0, s, t);
     return;
